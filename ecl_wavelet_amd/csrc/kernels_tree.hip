@@ -47,31 +47,36 @@ template <> struct CodeOf<8> { using type = uint64_t; };
 // bit `bit` of each of the 16/sizeof(T) codes of a 16-byte chunk, code k at bit k
 template <typename T>
 __device__ __forceinline__ uint32_t chunk_mask(const uint4& v, uint32_t bit) {
-  const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-  uint32_t m = 0;
   if constexpr (sizeof(T) == 1) {
-    // isolate the bit of each byte of a dword and gather the four bits into
-    // a nibble with one multiply (the partial products do not overlap)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t x = (d[k] >> bit) & 0x01010101u;
-      m |= ((x * 0x01020408u) >> 24 & 0xFu) << (4 * k);
-    }
+    // the bit of every byte stays where it is and a dot product with the
+    // weights 1, 2, .., 128 gathers eight of them (the sum is at most 255
+    // times 2^bit), so a chunk takes four ands, four v_dot4_u32_u8 and one
+    // shift of both halves
+    const uint32_t m = 0x01010101u << bit;
+    uint32_t lo = __builtin_amdgcn_udot4(v.x & m, 0x08040201u, 0u, false);
+    lo = __builtin_amdgcn_udot4(v.y & m, 0x80402010u, lo, false);
+    uint32_t hi = __builtin_amdgcn_udot4(v.z & m, 0x08040201u, 0u, false);
+    hi = __builtin_amdgcn_udot4(v.w & m, 0x80402010u, hi, false);
+    return (lo | (hi << 8)) >> bit;
   } else if constexpr (sizeof(T) == 2) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      m |= ((d[k] >> bit) & 1u) << (2 * k);
-      m |= ((d[k] >> (16 + bit)) & 1u) << (2 * k + 1);
-    }
+    // the codes' bytes that hold the bit, side by side, then as above
+    const uint32_t sel = bit < 8 ? 0x06040200u : 0x07050301u, b = bit & 7;
+    const uint32_t m = 0x01010101u << b;
+    const uint32_t x = __builtin_amdgcn_perm(v.y, v.x, sel) & m;
+    const uint32_t y = __builtin_amdgcn_perm(v.w, v.z, sel) & m;
+    return __builtin_amdgcn_udot4(y, 0x80402010u,
+                                  __builtin_amdgcn_udot4(x, 0x08040201u, 0u, false), false) >> b;
   } else if constexpr (sizeof(T) == 4) {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+    uint32_t m = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) m |= ((d[k] >> bit) & 1u) << k;
+    return m;
   } else {
     const uint64_t a = (static_cast<uint64_t>(v.y) << 32) | v.x;
     const uint64_t b = (static_cast<uint64_t>(v.w) << 32) | v.z;
-    m = static_cast<uint32_t>((a >> bit) & 1u) | (static_cast<uint32_t>((b >> bit) & 1u) << 1);
+    return static_cast<uint32_t>((a >> bit) & 1u) | (static_cast<uint32_t>((b >> bit) & 1u) << 1);
   }
-  return m;
 }
 
 // code k of a 16-byte chunk, by shifts (k is a constant after unrolling)
@@ -554,8 +559,21 @@ __global__ __launch_bounds__(256) void span_words_kernel(PassParams p) {
 // completes it: such words are written once with a plain store.  Only a
 // word that a workgroup shares with another (at the ends of its span, or
 // where the tiles' nodes change) is OR-ed in atomically.  One owner thread
-// per group (thread 4q) handles the partial first and last word of the
+// per group (thread 511 - q) handles the partial first and last word of the
 // group's run; all other threads write its full words.
+//
+// The partition and what bounds it.  A chunk that lies inside one group (all
+// but the one or two per group that hold its ends) looks up its two bases
+// once, is put in order of the level's bit by a table of byte permutations
+// (8 codes per lookup) before the scan's barrier, and then stores each code
+// at one of two running addresses: about 40 VALU instructions per 16 codes
+// where a base, a rank and two counters per code took 140.  At n = 6e9, sigma
+// = 256 the pass went from 15.4 to 12.5 ms (94 -> 56 VALU instructions per
+// code).  What is left is the LDS: every ds_write of a wave takes 4.3 cycles
+// whatever its width, 5.6 with the partition's bank conflicts (measured over
+// 24 waves per CU), so the seven byte stores per code alone fill 60% of the
+// time.  Wider stores would have to be aligned: an unaligned ds_write_b16 or
+// b32 takes about 65 cycles.
 //
 // Waves per SIMD that the tile's LDS allows (three, four, four workgroups
 // of eight waves per CU for 4, 2, 1 chunk rows): the register budget
@@ -579,13 +597,125 @@ constexpr uint32_t kNoCarry = 0xFF;
 __device__ __forceinline__ uint32_t low_mask(uint32_t nbits) {
   return nbits >= 32 ? 0xFFFFFFFFu : (1u << nbits) - 1u;
 }
-// 32 bits of the tile's bit string from bit sp on (zeros past its end)
-template <uint32_t T>
+// 32 bits of the tile's bit string from bit sp on (the string has a word
+// past its end, whose bits no caller uses)
 __device__ __forceinline__ uint32_t tile_bits(const uint32_t* bits, uint32_t sp) {
   const uint32_t sw = sp >> 5;
-  const uint64_t win = static_cast<uint64_t>(bits[sw]) |
-                       (sw + 1 < T / 32 ? static_cast<uint64_t>(bits[sw + 1]) << 32 : 0ull);
-  return static_cast<uint32_t>(win >> (sp & 31));
+  return __builtin_amdgcn_alignbit(bits[sw + 1], bits[sw], sp & 31);
+}
+
+// inclusive scan of lanes 0 .. 7 (the first half of a DPP row)
+__device__ __forceinline__ uint32_t first8_incl_scan_u32(uint32_t v) {
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xF, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xF, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xF, 0xF, false));
+  return v;
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(lane)));
+}
+
+// Codes of the chunks that hold the end of a group (not at the chunk's own
+// end), one lane each: lane x takes code x % E of the chunk holding the end
+// of group x / E, when no earlier group ends inside the same chunk.  s_hc[q
+// << gshift] is the end of group q - 1; the last one is the number of codes
+// present.
+// Returns the code's tile position, with the group's end from the chunk's
+// start in the high half, or kNoEdge.
+constexpr uint32_t kNoEdge = 0xFFFFFFFFu;
+constexpr uint32_t kNoBases = 0xFFFFFFFFu;  // two 16-bit bases are at most 2^15 each
+template <uint32_t E>
+__device__ __forceinline__ uint32_t edge_code(uint32_t x, uint32_t ngroups, uint32_t gshift,
+                                              uint32_t npres, const uint32_t* s_hc) {
+  const uint32_t q = x / E + 1;
+  if (q > ngroups) return kNoEdge;
+  const uint32_t end = s_hc[q << gshift], prev = s_hc[(q - 1) << gshift];
+  const uint32_t in_chunk = end % E, pos = (end & ~(E - 1)) + x % E;
+  const bool first = ((prev ^ end) & ~(E - 1)) != 0 || prev % E == 0;
+  return in_chunk != 0 && first && pos < npres ? pos | (in_chunk << 16) : kNoEdge;
+}
+
+// Sort tables of the partition: entry m of s_sort holds the v_perm selectors
+// that put 8 bytes (CW 1) or 4 halfwords (CW 2) in stable order of their
+// mask bits, zeros first.
+template <int CW> struct SortTable {
+  static constexpr uint32_t codes = CW == 1 ? 8 : 4;          // codes per entry
+  static constexpr uint32_t entries = CW <= 2 ? 1u << codes : 1;
+};
+template <int CW>
+__device__ __forceinline__ uint2 sort_entry(uint32_t m) {
+  uint64_t sel = 0;
+  uint32_t at = 0;
+#pragma unroll
+  for (uint32_t bit = 0; bit < 2; ++bit)
+#pragma unroll
+    for (uint32_t j = 0; j < SortTable<CW>::codes; ++j)
+      if (((m >> j) & 1u) == bit) {
+        const uint64_t bytes = CW == 1 ? j : (2 * j) | ((2 * j + 1) << 8);
+        sel |= bytes << (8 * CW * at);
+        ++at;
+      }
+  return make_uint2(static_cast<uint32_t>(sel), static_cast<uint32_t>(sel >> 32));
+}
+
+// The codes of each half of the chunk in stable order of their mask bits
+// (for split_chunk; 4- and 8-byte codes stay as they are)
+template <typename Code>
+__device__ __forceinline__ uint4 sort_chunk(const uint4& v, uint32_t mask, const uint2* sort) {
+  if constexpr (sizeof(Code) <= 2) {
+    constexpr uint32_t N = 8 / sizeof(Code);
+    const uint2 a = sort[mask & ((1u << N) - 1u)], b = sort[mask >> N];
+    return make_uint4(__builtin_amdgcn_perm(v.y, v.x, a.x), __builtin_amdgcn_perm(v.y, v.x, a.y),
+                      __builtin_amdgcn_perm(v.w, v.z, b.x), __builtin_amdgcn_perm(v.w, v.z, b.y));
+  } else {
+    return v;
+  }
+}
+
+// Stable one-bit split of a chunk whose codes belong to one group: the codes
+// with mask bit 0 go to out[z], out[z + 1], .. and those with bit 1 to
+// out[o], out[o + 1], ..  v comes from sort_chunk: each half is one run of
+// zeros and one of ones, its code j goes to z + j or to (o - zeros) + j, so
+// it costs a compare and a select, and its offset j rides in the store.
+template <typename Code>
+__device__ __forceinline__ void split_chunk(const uint4& v, uint32_t mask, uint32_t z, uint32_t o,
+                                            Code* out) {
+  if constexpr (sizeof(Code) <= 2) {
+    constexpr uint32_t N = 8 / sizeof(Code);
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h) {
+      const uint32_t ones = __popc((mask >> (N * h)) & ((1u << N) - 1u)), zeros = N - ones;
+      const uint32_t w[2] = {d[2 * h], d[2 * h + 1]};
+      const uint32_t oz = o - zeros;
+      // the odd bytes, moved down by one shift per dword: a store takes bits
+      // 0..7 or 16..23 of its register (the empty asm keeps the compiler
+      // from shifting by 24 once more)
+      uint32_t odd[2] = {w[0] >> 8, w[1] >> 8};
+      if constexpr (sizeof(Code) == 1) asm("" : "+v"(odd[0]), "+v"(odd[1]));
+#pragma unroll
+      for (uint32_t j = 0; j < N; ++j) {
+        Code* at = out + (j < zeros ? z : oz);
+        if constexpr (sizeof(Code) == 1) {
+          const uint32_t x = (j & 1) ? odd[j >> 2] : w[j >> 2];
+          at[j] = static_cast<Code>((j & 2) ? x >> 16 : x);
+        } else {
+          at[j] = static_cast<Code>((j & 1) ? w[j >> 1] >> 16 : w[j >> 1]);
+        }
+      }
+      z += zeros;
+      o += ones;
+    }
+  } else {
+    constexpr uint32_t N = 16 / sizeof(Code);
+#pragma unroll
+    for (uint32_t j = 0; j < N; ++j) {
+      const uint32_t b = (mask >> j) & 1u;
+      out[b ? o : z] = chunk_elem<Code>(v, j);
+      o += b;
+      z += b ^ 1u;
+    }
+  }
 }
 
 template <int CW, int ROWS>
@@ -599,10 +729,12 @@ void pass_kernel(PassParams p) {
   constexpr uint32_t T = kTileChunks * E;          // codes per tile
   constexpr uint32_t LPW = 32 / E;                 // lanes per 32-bit bit word
   static_assert(T <= 65535, "tile positions are kept in 16 bits");
+  // lanes for the codes of the chunks at the ends of up to 128 groups
+  constexpr uint32_t kEdgeIters = (128 * E + kPassThreads - 1) / kPassThreads;
   // the tile in the current level's order; rewritten in place by the
   // partition (every thread holds its chunks in registers by then)
   __shared__ uint4 s_buf[kTileChunks];
-  __shared__ uint32_t s_bits[kTileChunks * E / 32]; // level bits of the tile
+  __shared__ uint32_t s_bits[T / 32 + 1];          // level bits of the tile (one word past them)
   __shared__ uint32_t s_hc[kMaxBins + 1];          // codes of the tile with digit < x
   __shared__ uint64_t s_ec[kMaxBins + 1];          // node's codes with digit < x in earlier tiles
   __shared__ uint64_t s_pc[kMaxBins + 1];          // global start of (node, digit x)
@@ -611,16 +743,20 @@ void pass_kernel(PassParams p) {
   __shared__ uint64_t s_lw[8], s_lnw[8];           // word offset and words per level
   __shared__ uint64_t s_gR[kLevelGroups];          // group destination bit
   __shared__ uint32_t s_gSL[kLevelGroups];         // group tile start | length << 16
-  __shared__ uint32_t s_gw[kLevelGw];              // destination words before each group
+  __shared__ uint32_t s_gw[kLevelGw];              // full destination words before each group
   __shared__ uint16_t s_base[kLevelChildren];      // partition base per child
   __shared__ uint64_t s_cD[kLevelGroups];          // carried word (index into p.words)
   __shared__ uint32_t s_cV[kLevelGroups];          // its bits so far
   __shared__ uint8_t s_cLo[kLevelGroups];          // first of them; kNoCarry: none
   __shared__ uint8_t s_cHi[kLevelGroups];          // bit after the last of them
   __shared__ uint32_t s_even[8];                   // level's groups fit 512 >> i threads each
+  __shared__ uint2 s_sort[SortTable<CW>::entries]; // split_chunk's table
 
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid < kLevelGroups) s_cLo[tid] = kNoCarry;
+  if constexpr (CW <= 2) {
+    if (tid < SortTable<CW>::entries) s_sort[tid] = sort_entry<CW>(tid);
+  }
   const uint64_t span = p.tiles_per_wg ? p.tiles_per_wg : 1;
   const uint64_t tbeg = static_cast<uint64_t>(blockIdx.x) * span;
   const uint64_t tend = tbeg + span < p.num_tiles ? tbeg + span : p.num_tiles;
@@ -667,17 +803,25 @@ void pass_kernel(PassParams p) {
       s_lnw[lane] = p.node_lnw != nullptr ? p.node_lnw[g.node * 8ull + lane] : p.level_nwords[lane];
     }
   }
-  // ---- stage the tile
+  // ---- the tile's codes: level 0 takes them from registers; the later
+  // levels read the buffer, and so do the codes after the last whole chunk
   const Code* src = static_cast<const Code*>(
       (p.node_remap != nullptr && p.node_remap[g.node]) ? p.codes_out : p.codes);
+  uint4 v[kChunkRows];
+  if (g.len == T) {
 #pragma unroll
-  for (uint32_t r = 0; r < kChunkRows; ++r) {
-    const uint32_t c = r * kPassThreads + tid;
-    const uint32_t p0 = c * E;
-    uint4 q = make_uint4(0, 0, 0, 0);
-    if (p0 + E <= g.len) q = *reinterpret_cast<const uint4*>(src + g.start + p0);
-    else if (p0 < g.len) q = load_partial_chunk<Code>(src, g.start + p0, g.len - p0);
-    s_buf[c] = q;
+    for (uint32_t r = 0; r < kChunkRows; ++r)
+      v[r] = *reinterpret_cast<const uint4*>(src + g.start + (r * kPassThreads + tid) * E);
+  } else {
+#pragma unroll
+    for (uint32_t r = 0; r < kChunkRows; ++r) {
+      const uint32_t c = r * kPassThreads + tid;
+      const uint32_t p0 = c * E;
+      v[r] = make_uint4(0, 0, 0, 0);
+      if (p0 + E <= g.len) v[r] = *reinterpret_cast<const uint4*>(src + g.start + p0);
+      else if (p0 < g.len) v[r] = load_partial_chunk<Code>(src, g.start + p0, g.len - p0);
+      s_buf[c] = v[r];
+    }
   }
   // (digits >= nb never occur, so s_hc[x] and s_ec[x] for x >= nb hold the totals)
   __syncthreads();
@@ -702,7 +846,9 @@ void pass_kernel(PassParams p) {
         const uint32_t a = q << gshift, b = (q + 1) << gshift, m = a + (1u << (gshift - 1));
         const uint32_t len = s_hc[b] - s_hc[a];
         const uint64_t R = s_pc[a] + s_ec[b] - s_ec[a];
-        nw[j] = len ? static_cast<uint32_t>(((R & 31) + len + 31) >> 5) : 0u;
+        // full words of [R, R + len)
+        const uint32_t r5 = static_cast<uint32_t>(R) & 31u, last = (r5 + len) >> 5;
+        nw[j] = last > (r5 != 0 ? 1u : 0u) ? last - (r5 != 0 ? 1u : 0u) : 0u;
         ones[j] = s_hc[b] - s_hc[m];
         s_gR[grp_off(i) + q] = R;
         s_gSL[grp_off(i) + q] = s_hc[a] | (len << 16);
@@ -743,22 +889,65 @@ void pass_kernel(PassParams p) {
     const uint32_t npres = s_hc[s_thr[i]];            // tile codes present at level l0+i
     const uint32_t cbit = p.dshift + k - 1 - i;        // code bit of the level
     const uint32_t gshift = k - i;                     // digit >> gshift = group
+    const uint32_t ngroups = s_thr[i] >> gshift;
+    const bool partition = (i + 1 < k) || (p.dst != nullptr);
     // ---- level bits of the chunks; ones per chunk (16-bit field per row)
-    uint4 v[kChunkRows];
+    uint32_t mask[kChunkRows];
     uint64_t packed = 0;
+    if (i != 0) {
+#pragma unroll
+      for (uint32_t r = 0; r < kChunkRows; ++r) v[r] = s_buf[r * kPassThreads + tid];
+    }
 #pragma unroll
     for (uint32_t r = 0; r < kChunkRows; ++r) {
       const uint32_t c = r * kPassThreads + tid;
-      v[r] = s_buf[c];
       uint32_t mm = chunk_mask<Code>(v[r], cbit & 63);
       const uint32_t p0 = c * E;
-      if (p0 + E > npres) mm &= (p0 >= npres) ? 0u : ((1u << (npres - p0)) - 1u);
-      // 32-bit words of the tile's bit string: the chunks of LPW neighbouring lanes
-      uint32_t w32 = mm << (E * (lane % LPW));
+      if (npres != T && p0 + E > npres) mm &= (p0 >= npres) ? 0u : ((1u << (npres - p0)) - 1u);
+      mask[r] = mm;
+      if constexpr (E == 16) {
+        reinterpret_cast<uint16_t*>(s_bits)[c] = static_cast<uint16_t>(mm);
+      } else if constexpr (E == 8) {
+        reinterpret_cast<uint8_t*>(s_bits)[c] = static_cast<uint8_t>(mm);
+      } else {
+        // 32-bit words of the tile's bit string: the chunks of LPW neighbouring lanes
+        uint32_t w32 = mm << (E * (lane % LPW));
 #pragma unroll
-      for (uint32_t off = 1; off < LPW; off <<= 1) w32 |= __shfl_xor(w32, off, 64);
-      if (lane % LPW == 0) s_bits[p0 >> 5] = w32;
+        for (uint32_t off = 1; off < LPW; off <<= 1) w32 |= __shfl_xor(w32, off, 64);
+        if (lane % LPW == 0) s_bits[p0 >> 5] = w32;
+      }
       packed |= static_cast<uint64_t>(__popc(mm)) << (16 * r);
+    }
+    // For the partition, while the scan is under way: the chunks sorted by
+    // the level's bit, and the bases of the chunks that lie inside one group
+    // (their children's: child 2q takes the group's zeros, child 2q + 1 its
+    // ones).  No table is read between the partition's stores then, which
+    // the LDS counter would make wait for them.
+    const uint16_t* s_bs = s_base + child_off(i);
+    uint32_t bases[kChunkRows];
+    if (partition) {
+#pragma unroll
+      for (uint32_t r = 0; r < kChunkRows; ++r) {
+        const uint32_t p0 = (r * kPassThreads + tid) * E;
+        const uint32_t g0 = child_of<Code>(v[r], 0, cbit + 1, i);
+        const uint32_t g1 = child_of<Code>(v[r], E - 1, cbit + 1, i);
+        const uint32_t bb = *reinterpret_cast<const uint32_t*>(s_bs + 2 * g0);
+        bases[r] = p0 + E <= npres && g0 == g1 ? bb : kNoBases;
+        v[r] = sort_chunk<Code>(v[r], mask[r], s_sort);
+      }
+    }
+    // codes of chunks that hold a group's end (below): read before the
+    // partition rewrites the buffer
+    uint32_t edge[kEdgeIters];
+    Code ecode[kEdgeIters];
+    if (partition) {
+#pragma unroll
+      for (uint32_t e = 0; e < kEdgeIters; ++e)
+        if (e * kPassThreads < ngroups * E) {
+          edge[e] = edge_code<E>(e * kPassThreads + tid, ngroups, gshift, npres, s_hc);
+          if (edge[e] != kNoEdge)
+            ecode[e] = reinterpret_cast<const Code*>(s_buf)[edge[e] & 0xFFFFu];
+        }
     }
     // wave-local exclusive prefixes (fields stay below 2^16: no carries)
     const uint64_t incl = detail::wave_incl_scan_2x32(packed);
@@ -766,19 +955,22 @@ void pass_kernel(PassParams p) {
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     // ones before each of my chunks: earlier rows + earlier waves of my row,
-    // summed as packed 16-bit fields (one per row; no field overflows)
-    uint64_t all_waves = 0, waves_before = 0;
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(wave);
-#pragma unroll
-    for (uint32_t w = 0; w < kPassThreads / 64; ++w) {
-      const uint64_t x = s_wave[w];
-      all_waves += x;
-      if (w < wv) waves_before += x;
-    }
+    // as packed 16-bit fields (one per row; no field overflows).  The lanes
+    // hold the waves' sums; three DPP steps scan them and the scan's entries
+    // for this wave and for all waves come out as scalars.
     uint32_t O[kChunkRows];
+    uint32_t tot_ones = 0;
     {
-      uint32_t tot_ones = 0;
-      const uint64_t mine = waves_before + lex;
+      const uint32_t wv = __builtin_amdgcn_readfirstlane(wave);
+      static_assert(kPassThreads / 64 == 8, "one lane per wave in half a DPP row");
+      const uint64_t x = s_wave[lane & 7];
+      const uint32_t lo = first8_incl_scan_u32(static_cast<uint32_t>(x));
+      const uint32_t hi = first8_incl_scan_u32(static_cast<uint32_t>(x >> 32));
+      const uint64_t all_waves = (static_cast<uint64_t>(lane_value(hi, 7)) << 32) | lane_value(lo, 7);
+      uint64_t before = 0;
+      if (wv != 0)
+        before = (static_cast<uint64_t>(lane_value(hi, wv - 1)) << 32) | lane_value(lo, wv - 1);
+      const uint64_t mine = before + lex;
 #pragma unroll
       for (uint32_t r = 0; r < kChunkRows; ++r) {
         O[r] = tot_ones + (static_cast<uint32_t>(mine >> (16 * r)) & 0xFFFFu);
@@ -791,29 +983,29 @@ void pass_kernel(PassParams p) {
     // word lies inside the run, atomicOr on the two edge words shared with
     // neighbouring runs).
     {
-      const uint32_t ngroups = s_thr[i] >> gshift;
       const uint32_t* gw = s_gw + gw_off(i);
       const uint64_t* gR = s_gR + grp_off(i);
       const uint32_t* gSL = s_gSL + grp_off(i);
       const uint32_t total_words = gw[ngroups];
       const uint64_t lnw = s_lnw[i];
       uint32_t* words = p.words + s_lw[i];
-      // full words of the runs
+      // full words of the runs: word f of a run is the level's word
+      // ceil(R / 32) + f and starts at tile bit src0 + (-R mod 32) + 32 f
       if (s_even[i]) {
-        // group tid >> (9 - i), its words j = tid mod 2^(9-i) + m * 2^(9-i)
+        // group tid >> (9 - i), its words tid mod 2^(9-i) + m * 2^(9-i)
         const uint32_t tsh = 9u - i, q = tid >> tsh;
         if (q < ngroups) {
-          const uint32_t nwq = gw[q + 1] - gw[q];
+          uint32_t nf = gw[q + 1] - gw[q];
           const uint64_t R = gR[q];
-          const uint32_t sl = gSL[q];
-          const uint32_t src0 = sl & 0xFFFFu, len = sl >> 16;
-          const uint32_t r5 = static_cast<uint32_t>(R) & 31u;
-          for (uint32_t j = tid & ((1u << tsh) - 1u); j < nwq; j += 1u << tsh) {
-            if ((j == 0 && r5 != 0) || r5 + len < 32u * (j + 1)) continue;  // partial: owner's
-            const uint64_t D = (R >> 5) + j;
-            if (D >= lnw) atomicOr(p.err, 1u);
-            else words[D] = tile_bits<T>(s_bits, src0 + 32u * j - r5);
+          const uint64_t D = (R + 31) >> 5;
+          if (nf != 0 && D + nf > lnw) {
+            atomicOr(p.err, 1u);
+            nf = 0;
           }
+          uint32_t* out = words + D;
+          const uint32_t sp = (gSL[q] & 0xFFFFu) + (-static_cast<uint32_t>(R) & 31u);
+          for (uint32_t f = tid & ((1u << tsh) - 1u); f < nf; f += 1u << tsh)
+            out[f] = tile_bits(s_bits, sp + 32u * f);
         }
       } else
       for (uint32_t w = tid; w < total_words; w += kPassThreads) {
@@ -824,19 +1016,17 @@ void pass_kernel(PassParams p) {
           if (x <= w) { lo = mid; wlo = x; } else { hi = mid; }
         }
         const uint64_t R = gR[lo];
-        const uint32_t sl = gSL[lo];
-        const uint32_t src0 = sl & 0xFFFFu, len = sl >> 16;
-        const uint32_t j = w - wlo;                   // word of the run
-        const uint32_t r5 = static_cast<uint32_t>(R) & 31u;
-        if ((j == 0 && r5 != 0) || r5 + len < 32u * (j + 1)) continue;  // partial: owner's
-        const uint64_t D = (R >> 5) + j;
-        const uint32_t sp = src0 + 32u * j - r5;
+        const uint64_t D = ((R + 31) >> 5) + (w - wlo);
+        const uint32_t sp =
+            (gSL[lo] & 0xFFFFu) + (-static_cast<uint32_t>(R) & 31u) + 32u * (w - wlo);
         if (D >= lnw) atomicOr(p.err, 1u);
-        else words[D] = tile_bits<T>(s_bits, sp);
+        else words[D] = tile_bits(s_bits, sp);
       }
-      // partial first and last words: group q's owner, thread 4q
-      if ((tid & 3u) == 0 && (tid >> 2) < ngroups) {
-        const uint32_t q = tid >> 2;
+      // partial first and last words: group q's owner, thread 511 - q (the
+      // owners fill as few waves as they can, and not those of the group
+      // ends below)
+      if (kPassThreads - 1 - tid < ngroups) {
+        const uint32_t q = kPassThreads - 1 - tid;
         const uint32_t sl = gSL[q];
         const uint32_t src0 = sl & 0xFFFFu, len = sl >> 16;
         if (len != 0) {
@@ -857,7 +1047,7 @@ void pass_kernel(PassParams p) {
           if (r5 != 0 || len < 32u) {
             // first word: the run's bits [r5, min(32, r5 + len)) join the carry
             const uint32_t hn = len < 32u - r5 ? len : 32u - r5;
-            cur |= (tile_bits<T>(s_bits, src0) & low_mask(hn)) << r5;
+            cur |= (tile_bits(s_bits, src0) & low_mask(hn)) << r5;
             if (clo == kNoCarry) clo = r5;
             if (r5 + len >= 32u) {  // complete
               if (D0 >= lnw) atomicOr(p.err, 1u);
@@ -871,7 +1061,7 @@ void pass_kernel(PassParams p) {
           const uint32_t e5 = static_cast<uint32_t>(R + len) & 31u;
           if (r5 + len > 32u && e5 != 0) {
             // last word: bits [0, e5), carried into the next tile
-            cur = tile_bits<T>(s_bits, src0 + len - e5) & low_mask(e5);
+            cur = tile_bits(s_bits, src0 + len - e5) & low_mask(e5);
             clo = 0;
             chi = e5;
             s_cD[ci] = s_lw[i] + ((R + len) >> 5);
@@ -888,65 +1078,35 @@ void pass_kernel(PassParams p) {
         }
       }
     }
-    const bool partition = (i + 1 < k) || (p.dst != nullptr);
     if (!partition) break;
-    // ---- partition: child c of group c >> 1 takes its zeros (c even) or
-    // ones (c odd) in order from its base (level tables)
-    const uint16_t* s_bs = s_base + child_off(i);
+    // ---- partition: the chunks inside one group, then the codes of those
+    // that hold a group's end
     Code* both = reinterpret_cast<Code*>(s_buf);
-    const uint32_t cwidth = i + 1;  // child index = top i+1 digit bits
-    if (npres == T && i == 0) {
-      // one group, two children: the bases stay in registers
-      const uint32_t base0 = s_bs[0], base1 = s_bs[1];
 #pragma unroll
-      for (uint32_t r = 0; r < kChunkRows; ++r) {
-        const uint32_t p0 = (r * kPassThreads + tid) * E;
-        uint32_t o = O[r], z = p0 - O[r];
-#pragma unroll
-        for (uint32_t j = 0; j < E; ++j) {
-          const uint32_t b = child_of<Code>(v[r], j, cbit, 1);
-          both[(b ? base1 + o : base0 + z)] = chunk_elem<Code>(v[r], j);
-          o += b;
-          z += b ^ 1u;
-        }
-      }
-    } else if (npres == T) {
-      // every code of the tile is present at this level: no per-code tests
-#pragma unroll
-      for (uint32_t r = 0; r < kChunkRows; ++r) {
-        const uint32_t p0 = (r * kPassThreads + tid) * E;
-        uint32_t child[E], base[E];
-#pragma unroll
-        for (uint32_t j = 0; j < E; ++j) child[j] = child_of<Code>(v[r], j, cbit, cwidth);
-#pragma unroll
-        for (uint32_t j = 0; j < E; ++j) base[j] = s_bs[child[j]];
-        uint32_t o = O[r], z = p0 - O[r];
-#pragma unroll
-        for (uint32_t j = 0; j < E; ++j) {
-          const uint32_t b = child[j] & 1u;
-          both[base[j] + (b ? o : z)] = chunk_elem<Code>(v[r], j);
-          o += b;
-          z += b ^ 1u;
-        }
-      }
-    } else {
-#pragma unroll
-      for (uint32_t r = 0; r < kChunkRows; ++r) {
-        const uint32_t p0 = (r * kPassThreads + tid) * E;
-        if (p0 >= npres) continue;
-        uint32_t o = O[r], z = p0 - O[r];
-#pragma unroll
-        for (uint32_t j = 0; j < E; ++j) {
-          if (p0 + j < npres) {
-            const uint32_t child = child_of<Code>(v[r], j, cbit, cwidth);
-            const uint32_t b = child & 1u;
-            both[s_bs[child] + (b ? o : z)] = chunk_elem<Code>(v[r], j);
-            o += b;
-            z += b ^ 1u;
-          }
-        }
-      }
+    for (uint32_t r = 0; r < kChunkRows; ++r) {
+      const uint32_t p0 = (r * kPassThreads + tid) * E;
+      if (bases[r] != kNoBases)
+        split_chunk<Code>(v[r], mask[r], (bases[r] & 0xFFFFu) + p0 - O[r],
+                          (bases[r] >> 16) + O[r], both);
     }
+#pragma unroll
+    for (uint32_t e = 0; e < kEdgeIters; ++e)
+      if (e * kPassThreads < ngroups * E) {
+        if (edge[e] != kNoEdge) {
+          // ones before the group end inside the chunk (those before the next
+          // group are its zeros' base) less the chunk's ones from here to it,
+          // or plus those from it to here
+          const uint32_t q = (e * kPassThreads + tid) / E + 1;
+          const uint32_t pos = edge[e] & 0xFFFFu, in_chunk = edge[e] >> 16;
+          const uint32_t cm = s_bits[pos >> 5] >> (pos & 31 & ~(E - 1));
+          const uint32_t at_end = q < ngroups ? s_bs[2 * q] : tot_ones;
+          const uint32_t o = at_end - __popc(cm & ((1u << in_chunk) - 1u)) +
+                             __popc(cm & ((1u << (pos % E)) - 1u));
+          const uint32_t child =
+              static_cast<uint32_t>(static_cast<uint64_t>(ecode[e]) >> (cbit & 63)) & ((2u << i) - 1u);
+          both[s_bs[child] + ((child & 1u) ? o : pos - o)] = ecode[e];
+        }
+      }
     __syncthreads();
   }
 

@@ -1,0 +1,39 @@
+"""Construction at the edges of its tiles: text lengths around whole chunks
+and tiles, and symbol counts that put the ends of many, few, empty and tiny
+groups inside the 16-byte chunks of a level.  Every level's bits, count and
+node rank equals the oracle's tree over the same text."""
+import numpy as np
+import pytest
+
+from test_gpu_wavelet_tree import _check_structure_vs_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _text(kind, n, sigma, rng):
+    if kind == "uniform":
+        return rng.integers(0, sigma, n)
+    if kind == "rare":  # one symbol takes nearly everything, the others a few places
+        t = np.full(n, sigma // 2)
+        at = rng.integers(0, n, min(n, 3 * sigma))
+        t[at] = rng.integers(0, sigma, at.size)
+        return t
+    if kind == "sorted":  # whole tiles of one symbol
+        return np.sort(rng.integers(0, sigma, n))
+    return np.arange(n) * 7 % sigma  # "cycle": every group the same length
+
+
+@pytest.mark.parametrize("kind", ["uniform", "rare", "sorted", "cycle"])
+@pytest.mark.parametrize("dt,sigma", [(np.uint8, 2), (np.uint8, 4), (np.uint8, 20),
+                                      (np.uint8, 129), (np.uint8, 256), (np.uint16, 300),
+                                      (np.uint16, 1024), (np.uint32, 70000)])
+def test_tile_and_chunk_edges(gpu, dt, sigma, kind):
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(sigma)
+    tile = 32768 // np.dtype(dt).itemsize
+    for n in (1, 15, 16, 17, 33, tile - 1, tile, tile + 1, 2 * tile + 17):
+        if sigma > 65536 and n > tile:
+            continue
+        text = _text(kind, n, sigma, rng).astype(dt)
+        wt = WaveletTree(text, np.arange(sigma, dtype=dt))
+        _check_structure_vs_oracle(wt, text, sigma)
