@@ -881,17 +881,22 @@ struct BuildPlan {
   int cw = 1;
   uint32_t npasses = 1;
   std::vector<uint32_t> k, l0;  // levels per pass and first level
+  std::vector<int> w;           // bytes per code of each pass's input
 };
+int code_bytes(uint32_t bits) { return bits <= 8 ? 1 : bits <= 16 ? 2 : bits <= 32 ? 4 : 8; }
 BuildPlan plan_of(uint32_t L) {
   BuildPlan b;
-  b.cw = L <= 8 ? 1 : L <= 16 ? 2 : L <= 32 ? 4 : 8;
+  b.cw = code_bytes(L);
   b.npasses = (L + 7) / 8;
   b.k.resize(b.npasses);
   b.l0.resize(b.npasses);
+  b.w.resize(b.npasses);
   uint32_t acc = 0;
   for (uint32_t q = 0; q < b.npasses; ++q) {
     b.k[q] = L / b.npasses + (q < L % b.npasses ? 1u : 0u);
     b.l0[q] = acc;
+    // a later pass reads only the code bits below its first level
+    b.w[q] = code_bytes(L - acc);
     acc += b.k[q];
   }
   return b;
@@ -922,12 +927,12 @@ TreeMemory tree_memory(uint64_t n, uint64_t sigma, uint32_t L, int esize, bool h
   TreeMemory m;
   m.resident = per_level * L + scan + sigma * 64 + (n / 4096 + 4096) * 8 +
                10'000'000ull * 16;
-  // level order with padded nodes (the build's pad_cap)
-  const uint64_t pad = (n + (2 * sigma + 2) * (16 / b.cw)) * b.cw;
+  // level order with padded nodes (the build's pad_cap) of codes of w bytes
+  auto pad = [&](uint64_t w) { return (n + (2 * sigma + 2) * (16 / w)) * w; };
   m.text = host_text ? n * esize : 0;
-  m.x = identity ? 0 : (b.npasses > 2 ? pad : n * b.cw);
-  m.u = b.npasses > 1 ? pad : 0;
-  m.v = b.npasses > 2 && identity ? pad : 0;
+  m.x = identity ? 0 : (b.npasses > 2 ? pad(b.cw) : n * b.cw);
+  m.u = b.npasses > 1 ? pad(b.w[1]) : 0;
+  m.v = b.npasses > 2 && identity ? pad(b.w[2]) : 0;
   return m;
 }
 uint64_t tree_needed_bytes(uint64_t n, uint64_t sigma, uint32_t L, int esize, bool host_text) {
@@ -1126,8 +1131,7 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     const BuildPlan plan = plan_of(L);
     const int cw = plan.cw;
     const uint32_t rows = 4;
-    const uint64_t T = pass_tile_codes(cw, rows);   // codes per tile
-    const uint64_t E = 16 / cw;               // codes per 16 bytes
+    const uint64_t T0 = pass_tile_codes(cw, rows);  // codes per tile of the first pass
 
     // the passes read 16-byte vectors: a text that is its own code and is
     // aligned is read in place, anything else is mapped to codes first (a
@@ -1208,20 +1212,22 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     // scan for the largest pass, error flag, first pass digit starts and
     // thresholds, directory tables
     StagingBuf buf_x, buf_u, buf_v;
-    uint64_t max_tiles = (n + T - 1) / T;
+    uint64_t max_tiles = (n + T0 - 1) / T0;
     for (uint32_t q = 1; q < plan.npasses; ++q)
-      max_tiles = std::max<uint64_t>(max_tiles, n / T + (1ull << plan.l0[q]) + 1);
+      max_tiles = std::max<uint64_t>(max_tiles, n / pass_tile_codes(plan.w[q], rows) +
+                                                    (1ull << plan.l0[q]) + 1);
     const uint32_t kmax = plan.k[0];
-    const uint64_t pad_cap = n + (2 * sigma + 2) * E;  // level order with padded nodes
-    if (!identity) buf_x.alloc((plan.npasses > 2 ? pad_cap : n) * cw, x_host);
-    if (plan.npasses > 1) buf_u.alloc(pad_cap * cw, u_host);
-    if (plan.npasses > 2 && identity) buf_v.alloc(pad_cap * cw, v_host);
-    if ((!identity && (plan.npasses > 2 ? pad_cap : n) * cw != mem.x) ||
-        (plan.npasses > 1 ? pad_cap * cw : 0) != mem.u ||
-        (plan.npasses > 2 && identity ? pad_cap * cw : 0) != mem.v)
+    // codes of w bytes a level order with padded nodes holds
+    auto pad_cap = [&](uint64_t w) { return n + (2 * sigma + 2) * (16 / w); };
+    if (!identity) buf_x.alloc((plan.npasses > 2 ? pad_cap(cw) : n) * cw, x_host);
+    if (plan.npasses > 1) buf_u.alloc(pad_cap(plan.w[1]) * plan.w[1], u_host);
+    if (plan.npasses > 2 && identity) buf_v.alloc(pad_cap(plan.w[2]) * plan.w[2], v_host);
+    if ((!identity && (plan.npasses > 2 ? pad_cap(cw) : n) * cw != mem.x) ||
+        (plan.npasses > 1 ? pad_cap(plan.w[1]) * plan.w[1] : 0) != mem.u ||
+        (plan.npasses > 2 && identity ? pad_cap(plan.w[2]) * plan.w[2] : 0) != mem.v)
       throw Error(ECL_ERROR_INTERNAL, "code buffer sizes differ from the memory estimate");
     const uint32_t k0 = plan.k[0], nb0 = 1u << k0;
-    const uint64_t tiles0 = (n + T - 1) / T;
+    const uint64_t tiles0 = (n + T0 - 1) / T0;
     Scratch scr(device, s,
                 Scratch::units((max_tiles << kmax) * 4) +
                     Scratch::units(((max_tiles + 1) << kmax) * 8) +
@@ -1246,7 +1252,7 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     pp.code_table = wt->d_codes.as<uint64_t>();
     pp.cw = cw;
     pp.tile_rows = rows;
-    pp.tile_codes = static_cast<uint32_t>(T);
+    pp.tile_codes = static_cast<uint32_t>(T0);
     launch_fill_u32(d_err, 1, 0, s);
     pp.err = d_err;
     pp.hist = d_hist_t;
@@ -1308,8 +1314,11 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
       const uint32_t k = plan.k[q], l0 = plan.l0[q], nb = 1u << k;
       const uint64_t nodes = 1ull << l0;
       const bool last = q + 1 == plan.npasses;
+      const uint64_t T = pass_tile_codes(plan.w[q], rows);
       pp.k = k;
       pp.dshift = L - l0 - k;
+      pp.cw = plan.w[q];
+      pp.tile_codes = static_cast<uint32_t>(T);
       if (q > 0) {
         // node-aligned tiles over the padded level-l0 order
         std::vector<uint64_t> tstart;
@@ -1334,7 +1343,7 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
         h2d(d_tnode.ptr, tnode.data(), ntiles);
         h2d(d_tfirst.ptr, tfirst.data(), nodes + 1);
         pp.src = in_codes;
-        pp.src_esize = cw;
+        pp.src_esize = plan.w[q];
         pp.codes_out = nullptr;
         pp.codes = in_codes;
         pp.map_kind = 0;
@@ -1413,6 +1422,7 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
       if (!last) {
         next_size.assign(nodes * nb, 0);
         next_pstart.assign(nodes * nb, 0);
+        const uint64_t E = 16 / plan.w[q + 1];  // codes per 16 bytes
         uint64_t run = 0;
         for (uint64_t P = 0; P < nodes; ++P)
           for (uint32_t d = 0; d < nb; ++d) {
@@ -1421,7 +1431,7 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
             next_pstart[Q] = run;
             run += (next_size[Q] + E - 1) / E * E;
           }
-        if (run > pad_cap) throw Error(ECL_ERROR_INTERNAL, "level buffer too small");
+        if (run > pad_cap(plan.w[q + 1])) throw Error(ECL_ERROR_INTERNAL, "level buffer too small");
         d_obase = DevBuf(next_pstart.size() * 8);
         h2d(d_obase.ptr, next_pstart.data(), next_pstart.size());
         // outputs alternate between two buffers that differ from the input
@@ -1429,7 +1439,8 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
         pp.obase = d_obase.as<uint64_t>();
       }
       pp.dst = out_buf;
-      pp.dst_cap = out_buf ? pad_cap : 0;
+      pp.dst_cw = last ? 0 : plan.w[q + 1];
+      pp.dst_cap = out_buf ? pad_cap(plan.w[q + 1]) : 0;
       pp.words = ba->words();
       for (uint32_t i = 0; i < k; ++i) {
         pp.level_word[i] = ba->offsets[l0 + i];

@@ -182,6 +182,7 @@ struct PassParams {
   const uint64_t* obase;      // [nodes][2^k] padded start of (node, digit) in dst
   const uint16_t* thr;        // [nodes][k + 1] first absent digit per level
   void* dst;                  // level-(l0+k) codes, or nullptr on the last pass
+  int dst_cw;                 // bytes per code of dst: the code bits of the levels left
   uint64_t dst_cap;           // codes dst can hold
   uint32_t* words;            // bit array words
   uint64_t level_word[8];     // word offset of levels l0 .. l0+k-1

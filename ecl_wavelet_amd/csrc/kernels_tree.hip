@@ -718,6 +718,22 @@ __device__ __forceinline__ void split_chunk(const uint4& v, uint32_t mask, uint3
   }
 }
 
+// The tile's first nout codes, grouped by digit, to the next pass's input:
+// the code at tile position x with digit d goes to place base[d] + x.
+template <typename Code, typename Out>
+__device__ __forceinline__ void write_codes(const PassParams& p, const uint4* buf,
+                                            const uint64_t* base, uint32_t nout, uint32_t nb) {
+  const Code* cb = reinterpret_cast<const Code*>(buf);
+  Out* dst = static_cast<Out*>(p.dst);
+  for (uint32_t x = threadIdx.x; x < nout; x += kPassThreads) {
+    const Code c = cb[x];
+    const uint32_t d = static_cast<uint32_t>(static_cast<uint64_t>(c) >> p.dshift) & (nb - 1);
+    const uint64_t o = base[d] + x;
+    if (o < p.dst_cap) dst[o] = static_cast<Out>(c);
+    else atomicOr(p.err, 1u);
+  }
+}
+
 template <int CW, int ROWS>
 __global__ __launch_bounds__(kPassThreads)
 __attribute__((amdgpu_waves_per_eu(PassOcc<ROWS>::waves)))
@@ -1119,15 +1135,11 @@ void pass_kernel(PassParams p) {
       s_pc[d] = ob[d] + (s_ec[d + 1] - s_ec[d]) - s_hc[d];
     __syncthreads();
     const uint32_t nout = s_hc[s_thr[k]];
-    const Code* cb = reinterpret_cast<const Code*>(s_buf);
-    Code* dst = static_cast<Code*>(p.dst);
-    const uint32_t dmask = nb - 1;
-    for (uint32_t x = tid; x < nout; x += kPassThreads) {
-      const Code c = cb[x];
-      const uint32_t d = static_cast<uint32_t>(static_cast<uint64_t>(c) >> p.dshift) & dmask;
-      const uint64_t o = s_pc[d] + x;
-      if (o < p.dst_cap) dst[o] = c;
-      else atomicOr(p.err, 1u);
+    switch (p.dst_cw) {  // as narrow as the code bits of the levels left
+      case 1: write_codes<Code, uint8_t>(p, s_buf, s_pc, nout, nb); break;
+      case 2: if constexpr (CW >= 2) write_codes<Code, uint16_t>(p, s_buf, s_pc, nout, nb); break;
+      case 4: if constexpr (CW >= 4) write_codes<Code, uint32_t>(p, s_buf, s_pc, nout, nb); break;
+      default: if constexpr (CW == 8) write_codes<Code, uint64_t>(p, s_buf, s_pc, nout, nb); break;
     }
   }
   __syncthreads();  // the next tile rewrites the tables and the buffer
