@@ -1231,13 +1231,11 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     Scratch scr(device, s,
                 Scratch::units((max_tiles << kmax) * 4) +
                     Scratch::units(((max_tiles + 1) << kmax) * 8) +
-                    Scratch::units(scan_partial_entries(max_tiles, kmax) * 8) +
                     Scratch::units(4) + Scratch::units((nb0 + 1) * 8) +
                     Scratch::units((k0 + 1) * 2) +
                     directory_scratch_bytes(std::vector<uint64_t>(L, n)));
     uint32_t* d_hist_t = scr.carve<uint32_t>(max_tiles << kmax);
     uint64_t* d_excl = scr.carve<uint64_t>((max_tiles + 1) << kmax);
-    uint64_t* d_partial = scr.carve<uint64_t>(scan_partial_entries(max_tiles, kmax));
     uint32_t* d_err = scr.carve<uint32_t>(1);
     uint64_t* d_pc0 = scr.carve<uint64_t>(nb0 + 1);
     uint16_t* d_thr0 = scr.carve<uint16_t>(k0 + 1);
@@ -1257,7 +1255,6 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     pp.err = d_err;
     pp.hist = d_hist_t;
     pp.excl = d_excl;
-    pp.partial = d_partial;
 
     // ---- pass 0 digit counts (the whole text is one node)
     pp.src = d_text;

@@ -175,7 +175,7 @@ struct ForestBuild {
   uint32_t rows = 1;
   uint64_t ntiles = 0, blocks = 0, chunks = 0, meta_at = 0;
   uint32_t N = 0, ndesc = 0;
-  DevBuf d_x, d_tstart, d_tlen, d_tnode, d_tfirst, d_remap, d_lut, d_hist, d_excl, d_partial,
+  DevBuf d_x, d_tstart, d_tlen, d_tnode, d_tfirst, d_remap, d_lut, d_hist, d_excl,
       d_err, d_rows, d_pc, d_thr, d_nk, d_lw, d_lnw, d_jobs, d_shapes, d_code, d_len, d_node,
       d_node_level, d_desc, d_blk, d_lvptr;
   PassParams pp{};
@@ -284,7 +284,6 @@ std::shared_ptr<ForestBuild> make_build(ecl_forest_t* f, uint32_t rows) {
   h2d(B->d_lut.ptr, lut.data(), N * 256);
   B->d_hist = DevBuf(B->ntiles * kRow * 4);
   B->d_excl = DevBuf((B->ntiles + 1) * kRow * 8);
-  B->d_partial = DevBuf(scan_partial_entries(B->ntiles, 8) * 8);
   B->d_err = DevBuf(4);
   B->d_rows = DevBuf((N + 1) * kRow * 8);
   B->d_pc = DevBuf(N * (kRow + 1) * 8);
@@ -424,7 +423,6 @@ std::shared_ptr<ForestBuild> make_build(ecl_forest_t* f, uint32_t rows) {
   pp.node_first_tile = B->d_tfirst.as<uint32_t>();
   pp.hist = B->d_hist.as<uint32_t>();
   pp.excl = B->d_excl.as<uint64_t>();
-  pp.partial = B->d_partial.as<uint64_t>();
   pp.err = B->d_err.as<uint32_t>();
   pp.node_remap = any_remap ? B->d_remap.as<uint8_t>() : nullptr;
   pp.node_lut = B->d_lut.as<uint8_t>();

@@ -177,7 +177,6 @@ struct PassParams {
   const uint32_t* node_first_tile;   // [nodes + 1], nullptr for uniform tiles
   uint32_t* hist;             // [tiles][2^k] digit counts per tile
   uint64_t* excl;             // [tiles + 1][2^k] exclusive column scan
-  uint64_t* partial;          // scan scratch, scan_partial_entries() u64
   const uint64_t* pc;         // [nodes][2^k + 1] global start of (node, digit)
   const uint64_t* obase;      // [nodes][2^k] padded start of (node, digit) in dst
   const uint16_t* thr;        // [nodes][k + 1] first absent digit per level
@@ -202,7 +201,6 @@ struct PassParams {
   uint32_t tiles_per_wg;
 };
 uint64_t pass_tile_codes(int cw, uint32_t rows);    // codes per tile
-uint64_t scan_partial_entries(uint64_t tiles, uint32_t k);
 void launch_tile_hist(const PassParams& p, hipStream_t s);
 void launch_tile_scan(const PassParams& p, hipStream_t s);
 void launch_pass(const PassParams& p, hipStream_t s);

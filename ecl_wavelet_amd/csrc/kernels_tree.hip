@@ -376,32 +376,41 @@ __global__ __launch_bounds__(kPassThreads) void tile_hist_small_kernel(PassParam
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive column scan of the tile histograms, in blocks of 256 tiles:
-//  partial[b][d] = sum of block b  ->  exclusive over blocks  ->  excl rows.
-constexpr uint32_t kScanTiles = 256;
+// Exclusive column scan of the tile histograms, in blocks of tiles:
+//  sum of block b  ->  exclusive over blocks  ->  excl rows; until the last
+// step a block's value sits in the excl row of its first tile, which is where
+// it ends.
+// Blocks of 32 tiles (more where a workgroup's 256 threads span more rows of
+// few bins): with 256 a table of 3*10^4 tiles filled only 119 workgroups, and
+// each thread's 256 loads in a row were bound by latency (n = 5e8, 256 bins:
+// 98 + 5 + 112 us for the three kernels; 32 tiles: 17 + 12 + 16 us).
+__host__ __device__ constexpr uint32_t scan_tiles(uint32_t nb) { return nb >= 8 ? 32 : 256 / nb; }
 
 __global__ __launch_bounds__(256) void scan_partial_kernel(const uint32_t* __restrict__ hist,
                                                            uint64_t tiles, uint32_t nb,
-                                                           uint64_t* __restrict__ partial) {
+                                                           uint64_t* __restrict__ excl) {
   __shared__ uint64_t s[256];
   const uint32_t tid = threadIdx.x;
   const uint32_t rows = 256 / nb, col = tid % nb, r0 = tid / nb;
-  const uint64_t t0 = blockIdx.x * static_cast<uint64_t>(kScanTiles);
-  const uint64_t t1 = (t0 + kScanTiles < tiles) ? t0 + kScanTiles : tiles;
+  const uint32_t bt = scan_tiles(nb);
+  const uint64_t t0 = blockIdx.x * static_cast<uint64_t>(bt);
+  const uint64_t t1 = (t0 + bt < tiles) ? t0 + bt : tiles;
   uint64_t sum = 0;
+#pragma unroll 8
   for (uint64_t t = t0 + r0; t < t1; t += rows) sum += hist[t * nb + col];
   s[tid] = sum;
   __syncthreads();
   if (tid < nb) {
     uint64_t tot = 0;
     for (uint32_t r = 0; r < rows; ++r) tot += s[r * nb + tid];
-    partial[blockIdx.x * static_cast<uint64_t>(nb) + tid] = tot;
+    excl[t0 * nb + tid] = tot;
   }
 }
 
 // one workgroup per digit column: exclusive scan of the block sums in place
-__global__ __launch_bounds__(256) void scan_blocks_kernel(uint64_t* __restrict__ partial,
+__global__ __launch_bounds__(256) void scan_blocks_kernel(uint64_t* __restrict__ excl,
                                                           uint64_t nblk, uint32_t nb) {
+  const uint64_t stride = static_cast<uint64_t>(scan_tiles(nb)) * nb;
   __shared__ uint64_t s_wave[4];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t col = blockIdx.x;
@@ -409,7 +418,8 @@ __global__ __launch_bounds__(256) void scan_blocks_kernel(uint64_t* __restrict__
   const uint64_t b0 = tid * per;
   const uint64_t b1 = (b0 + per < nblk) ? b0 + per : nblk;
   uint64_t sum = 0;
-  for (uint64_t b = b0; b < b1; ++b) sum += partial[b * nb + col];
+#pragma unroll 4
+  for (uint64_t b = b0; b < b1; ++b) sum += excl[b * stride + col];
   uint64_t incl = sum;
 #pragma unroll
   for (uint32_t off = 1; off < 64; off <<= 1) {
@@ -421,37 +431,40 @@ __global__ __launch_bounds__(256) void scan_blocks_kernel(uint64_t* __restrict__
   uint64_t run = incl - sum;
   for (uint32_t w = 0; w < wave; ++w) run += s_wave[w];
   for (uint64_t b = b0; b < b1; ++b) {
-    const uint64_t x = partial[b * nb + col];
-    partial[b * nb + col] = run;
+    const uint64_t x = excl[b * stride + col];
+    excl[b * stride + col] = run;
     run += x;
   }
 }
 
 // excl[t][d] = codes with digit d in tiles < t; row `tiles` holds the totals
 __global__ __launch_bounds__(256) void scan_final_kernel(const uint32_t* __restrict__ hist,
-                                                         const uint64_t* __restrict__ partial,
-                                                         uint64_t tiles, uint32_t nb,
-                                                         uint64_t* __restrict__ excl) {
+                                                         uint64_t tiles, uint32_t nb, uint64_t* excl) {
   __shared__ uint64_t s[256];
   const uint32_t tid = threadIdx.x;
   const uint32_t rows = 256 / nb, col = tid % nb, r0 = tid / nb;
-  const uint32_t seg = kScanTiles / rows;  // consecutive tiles per thread
+  const uint32_t bt = scan_tiles(nb), seg = bt / rows;  // consecutive tiles per thread
   const uint64_t blk = blockIdx.x;
-  const uint64_t t0 = blk * kScanTiles + static_cast<uint64_t>(r0) * seg;
+  const uint64_t t0 = blk * bt + static_cast<uint64_t>(r0) * seg;
   uint64_t sum = 0;
-  for (uint32_t j = 0; j < seg; ++j)
-    if (t0 + j < tiles) sum += hist[(t0 + j) * nb + col];
+  if (rows > 1) {
+#pragma unroll 8
+    for (uint32_t j = 0; j < seg; ++j)
+      if (t0 + j < tiles) sum += hist[(t0 + j) * nb + col];
+  }
   s[tid] = sum;
+  uint64_t run = excl[blk * bt * nb + col];  // rewritten (with the same value) below
   __syncthreads();
-  uint64_t run = partial[blk * nb + col];
   for (uint32_t r = 0; r < r0; ++r) run += s[r * nb + col];
+#pragma unroll 8
   for (uint32_t j = 0; j < seg; ++j) {
     const uint64_t t = t0 + j;
-    if (t >= tiles) break;
-    excl[t * nb + col] = run;
-    run += hist[t * nb + col];
+    if (t < tiles) {
+      excl[t * nb + col] = run;
+      run += hist[t * nb + col];
+    }
   }
-  const uint64_t last_blk = (tiles - 1) / kScanTiles;
+  const uint64_t last_blk = (tiles - 1) / bt;
   if (blk == last_blk && r0 == rows - 1) excl[tiles * nb + col] = run;
 }
 
@@ -1229,22 +1242,18 @@ void launch_tile_hist(const PassParams& p, hipStream_t s) {
   ECL_HIP(hipGetLastError());
 }
 
-uint64_t scan_partial_entries(uint64_t tiles, uint32_t k) {
-  return ((tiles + kScanTiles - 1) / kScanTiles) << k;
-}
-
 void launch_tile_scan(const PassParams& p, hipStream_t s) {
   if (p.num_tiles == 0) return;
   ProfScope ps(K_TILE_SCAN, s);
   const uint32_t nb = p.row_bins ? p.row_bins : (1u << p.k);  // row stride
-  const uint64_t nblk = (p.num_tiles + kScanTiles - 1) / kScanTiles;
+  const uint64_t nblk = (p.num_tiles + scan_tiles(nb) - 1) / scan_tiles(nb);
   hipLaunchKernelGGL(scan_partial_kernel, dim3(static_cast<uint32_t>(nblk)), dim3(256), 0, s,
-                     p.hist, p.num_tiles, nb, p.partial);
+                     p.hist, p.num_tiles, nb, p.excl);
   ECL_HIP(hipGetLastError());
-  hipLaunchKernelGGL(scan_blocks_kernel, dim3(nb), dim3(256), 0, s, p.partial, nblk, nb);
+  hipLaunchKernelGGL(scan_blocks_kernel, dim3(nb), dim3(256), 0, s, p.excl, nblk, nb);
   ECL_HIP(hipGetLastError());
   hipLaunchKernelGGL(scan_final_kernel, dim3(static_cast<uint32_t>(nblk)), dim3(256), 0, s,
-                     p.hist, p.partial, p.num_tiles, nb, p.excl);
+                     p.hist, p.num_tiles, nb, p.excl);
   ECL_HIP(hipGetLastError());
 }
 
