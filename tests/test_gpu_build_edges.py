@@ -37,3 +37,16 @@ def test_tile_and_chunk_edges(gpu, dt, sigma, kind):
         text = _text(kind, n, sigma, rng).astype(dt)
         wt = WaveletTree(text, np.arange(sigma, dtype=dt))
         _check_structure_vs_oracle(wt, text, sigma)
+
+
+@pytest.mark.parametrize("sigma", [4, 20, 75, 200])
+def test_mapped_bytes_edges(gpu, sigma):
+    """Byte alphabets that are not 0..sigma-1 are mapped by table while the
+    tiles are counted: whole and partial chunks, and batches of four chunks."""
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(sigma)
+    alphabet = np.sort(rng.permutation(256)[:sigma]).astype(np.uint8)
+    for n in (1, 15, 17, 8191, 8192, 8193, 32768 + 16 * 512 * 3 + 5):
+        sym = rng.integers(0, sigma, n)
+        wt = WaveletTree(alphabet[sym], alphabet)
+        _check_structure_vs_oracle(wt, sym.astype(np.uint8), sigma)
