@@ -285,7 +285,7 @@ struct QuadBuildParams {
   // their second bits in order from z and whose ones from o
   const uint8_t* lut;
 };
-constexpr uint32_t kQuadWgInfo = 6;
+constexpr uint32_t kQuadWgInfo = 9;
 uint64_t quad_build_workgroups(uint64_t nlines);
 void launch_quad_lines(const QuadBuildParams& qp, hipStream_t s);
 // The quad lines and quad select lines of many quad levels (a forest's) in

@@ -822,10 +822,7 @@ void launch_multi_select_lines(const SelLinesJob* jobs, const uint64_t* wg_start
 // with o ones and z zeros of level 2q before it in its node has its level
 // 2q + 1 bit at S_N + z (bit 0) or S_N + Z_N + o (bit 1): a word of 32
 // positions inside one node takes its second bits from two contiguous runs
-// of level 2q + 1.  Line headers: the d's before position P are the d's
-// before its node (CD) plus, for d = 1 and 3, the ones of level 2q + 1 in
-// the two runs up to P (two ranks), and for d = 0 and 2 the rest of the
-// node's zeros and ones before P.
+// of level 2q + 1.
 // A workgroup builds kQuadLinesPerWg lines in LDS and writes them out
 // contiguously.
 constexpr uint32_t kQuadLinesPerWg = 64;
@@ -862,18 +859,32 @@ __device__ __forceinline__ uint64_t quad_node_from(const uint64_t* S, uint64_t n
   return lo;
 }
 
+// bits [x, x + 32) of a bit string in LDS that has a word past its end
+__device__ __forceinline__ uint32_t lds_bits32(const uint32_t* w, uint32_t x) {
+  return __builtin_amdgcn_alignbit(w[(x >> 5) + 1], w[x >> 5], x & 31);
+}
+
 // Thread t takes the 4 words (128 positions) from word 4t of the
 // workgroup's range; a block scan of their ones gives every word's rank from
 // one directory rank at the range's start, and the node search runs once per
-// workgroup (a thread searches only past a node start).
+// workgroup (a thread searches only past a node start).  A range inside one
+// node (nearly all) stages its two runs of level 2q + 1 in LDS with
+// coalesced loads; fetching each word's two windows from global memory had
+// taken 16 scattered loads per thread.  The line headers are the counts
+// before the range (quad_wg_kernel) plus a block scan of the digits built,
+// in place of two directory ranks per line.  Per level of n = 2e9: 617 -> 372
+// us (floor 235 us for the 1.07 GB read and written).
 __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_t blk) {
   constexpr uint32_t kWords = kQuadLinesPerWg * kQuadWordsPerLine;  // 896
+  static_assert(kWords <= 4 * 256, "four words per thread");
   __shared__ __align__(16) uint32_t s_lines[kQuadLinesPerWg * 32];
-  __shared__ uint32_t s_wrank[kWords];  // ones of level 2q before each word, from the range start
-  __shared__ uint32_t s_wave[4];
+  // the two runs: their bits are at most the range's, each with an unaligned
+  // start and end and a word past the end
+  __shared__ uint32_t s_runs[kWords + 6];
+  __shared__ uint32_t s_wave[4], s_wave13[4];
   // from quad_wg_kernel: ones of level 2q before the range, the node holding
   // its start (node0), node0's start and end, the ones of level 2q before
-  // node0 and the zeros in it
+  // node0 and the zeros in it, the digits 0, 1 and 2 before the range
   __shared__ uint64_t s_info[kQuadWgInfo];
   __shared__ __align__(16) uint8_t s_lut[4096];
   reinterpret_cast<uint4*>(s_lut)[threadIdx.x] =
@@ -899,64 +910,55 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
     }
   }
   const uint32_t pc = __popc(a4[0]) + __popc(a4[1]) + __popc(a4[2]) + __popc(a4[3]);
-  uint32_t incl = pc;
-#pragma unroll
-  for (uint32_t off = 1; off < 64; off <<= 1) {
-    const uint32_t y = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += y;
-  }
+  const uint32_t incl = detail::wave_incl_scan_u32(pc);
   if (lane == 63) s_wave[wave] = incl;
   if (tid < kQuadWgInfo) s_info[tid] = detail::gld(qp.wg_info, blk * kQuadWgInfo + tid);
   __syncthreads();
-  uint32_t run = incl - pc;
-  for (uint32_t w = 0; w < wave; ++w) run += s_wave[w];
-  for (uint32_t i = 0; i < 4; ++i) {
-    if (4 * tid + i < nwords) s_wrank[4 * tid + i] = run;
-    run += __popc(a4[i]);
-  }
+  uint32_t run0 = incl - pc;  // ones of the range before this thread's words
+  for (uint32_t w = 0; w < wave; ++w) run0 += s_wave[w];
   const uint64_t rank0 = s_info[0], node0 = s_info[1];
   const uint64_t SN0 = s_info[2], SN10 = s_info[3], OB0 = s_info[4], ZN0 = s_info[5];
+  // the range's first position, its positions and the ones among them
+  const uint64_t Pr = 32 * k0;
+  const uint32_t len = Pr < n ? static_cast<uint32_t>(n - Pr < 32ull * nwords ? n - Pr : 32ull * nwords) : 0u;
+  const uint32_t ones = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+  // one node: the zeros' run of level 2q + 1 starts at bit zx, the ones' at ox
+  const bool inside = len != 0 && Pr + len <= SN10;
+  const uint64_t o00 = rank0 - OB0, z00 = (Pr - SN0) - o00;
+  const uint64_t zx = SN0 + z00, ox = SN0 + ZN0 + o00;
+  const uint32_t zsh = static_cast<uint32_t>(zx) & 31u, osh = static_cast<uint32_t>(ox) & 31u;
+  const uint32_t nzw = (zsh + (len - ones) + 31) / 32 + 1, now = (osh + ones + 31) / 32 + 1;
+  if (inside) {
+    for (uint32_t i = tid; i < nzw + now; i += blockDim.x) {
+      const uint64_t k = i < nzw ? (zx >> 5) + i : (ox >> 5) + (i - nzw);
+      s_runs[i] = k < nw ? detail::gld(B, k) : 0u;
+    }
+  }
   __syncthreads();
-  // digits: 32 positions per word.  Words inside node0 (nearly all) take its
-  // parameters from LDS and fetch their two runs of level 2q + 1 first, all
-  // four words' runs at once; the others go the general way.
-  uint32_t zb[4], ob[4];
-  bool fast[4];
+  // digits: 32 positions per word, and the digits 1 and 3 among them
+  uint32_t c13[4] = {0u, 0u, 0u, 0u};  // digit 1 | digit 3 << 16
+  uint32_t run = run0;                 // ones of the range before the word
 #pragma unroll
   for (uint32_t i = 0; i < 4; ++i) {
     const uint32_t w = 4 * tid + i;
-    const uint64_t P0 = 32 * (k0 + w);
-    fast[i] = false;
-    zb[i] = ob[i] = 0;
-    if (w < nwords && P0 < n) {
-      const uint32_t valid = n - P0 < 32 ? static_cast<uint32_t>(n - P0) : 32u;
-      if (P0 + valid <= SN10) {
-        const uint64_t o0 = rank0 + s_wrank[w] - OB0;
-        const uint64_t z0 = (P0 - SN0) - o0;
-        zb[i] = bits32(B, nw, SN0 + z0);
-        ob[i] = bits32(B, nw, SN0 + ZN0 + o0);
-        fast[i] = true;
-      }
-    }
-  }
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t w = 4 * tid + i;
     if (w >= nwords) break;
-    const uint64_t P0 = 32 * (k0 + w);
-    uint64_t D = 0;
-    if (P0 < n) {
-      const uint32_t valid = n - P0 < 32 ? static_cast<uint32_t>(n - P0) : 32u;
+    const uint64_t P0 = Pr + 32ull * w;
+    uint32_t Dlo = 0, Dhi = 0;
+    if (32 * w < len) {
+      const uint32_t valid = len - 32 * w < 32 ? len - 32 * w : 32u;
       const uint32_t a = a4[i];  // bits past n are zero
-      const uint64_t rA = rank0 + s_wrank[w];  // ones of level 2q before P0
-      uint32_t zbi = zb[i], obi = ob[i];
-      bool one_node = fast[i];
+      uint32_t zbi = 0, obi = 0;
+      bool one_node = inside;
       uint64_t N = node0, SN = SN0, SN1 = SN10;
-      if (!one_node) {
+      if (inside) {
+        zbi = lds_bits32(s_runs, zsh + 32 * w - run);
+        obi = lds_bits32(s_runs + nzw, osh + run);
+      } else {
         N = quad_node_from(qp.S, qp.nodes, node0, P0);
         SN = detail::gld(qp.S, N);
         SN1 = detail::gld(qp.S, N + 1);
         if (P0 + valid <= SN1) {
-          const uint64_t o0 = rA - (cd(N, 2) + cd(N, 3));
+          const uint64_t o0 = rank0 + run - (cd(N, 2) + cd(N, 3));
           const uint64_t z0 = (P0 - SN) - o0;
           const uint64_t ZN = (cd(N + 1, 0) - cd(N, 0)) + (cd(N + 1, 1) - cd(N, 1));
           zbi = bits32(B, nw, SN + z0);
@@ -970,17 +972,23 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
         uint32_t iz = 0, io = 0;
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-          const uint32_t a4 = (a >> (4 * k)) & 15u;
+          const uint32_t ak = (a >> (4 * k)) & 15u;
           const uint32_t z4 = (zbi >> iz) & 15u, o4 = (obi >> io) & 15u;
-          D |= static_cast<uint64_t>(s_lut[a4 | (z4 << 4) | (o4 << 8)]) << (8 * k);
-          const uint32_t c = __popc(a4);
+          const uint32_t d = s_lut[ak | (z4 << 4) | (o4 << 8)];
+          if (k < 4) Dlo |= d << (8 * k);
+          else Dhi |= d << (8 * (k - 4));
+          const uint32_t c = __popc(ak);
           io += c;
           iz += 4u - c;
         }
         // positions past n (the last word) hold no digits
-        if (valid < 32) D &= (1ull << (2 * valid)) - 1;
+        if (valid < 32) {
+          Dlo &= valid >= 16 ? 0xFFFFFFFFu : (1u << (2 * valid)) - 1;
+          Dhi &= valid > 16 ? (1u << (2 * (valid - 16))) - 1 : 0u;
+        }
       } else {
         // the word crosses node starts: position by position
+        uint64_t D = 0;
         uint32_t before = 0;  // ones of the word before position j
         for (uint32_t j = 0; j < valid; ++j) {
           const uint64_t pos = P0 + j;
@@ -989,7 +997,7 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
             SN = SN1;
             SN1 = detail::gld(qp.S, N + 1);
           }
-          const uint64_t o = rA + before - (cd(N, 2) + cd(N, 3));
+          const uint64_t o = rank0 + run + before - (cd(N, 2) + cd(N, 3));
           const uint64_t z = (pos - SN) - o;
           const uint64_t ZN = (cd(N + 1, 0) - cd(N, 0)) + (cd(N + 1, 1) - cd(N, 1));
           const uint32_t aj = (a >> j) & 1u;
@@ -998,42 +1006,47 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
           D |= static_cast<uint64_t>((aj << 1) | bj) << (2 * j);
           before += aj;
         }
+        Dlo = static_cast<uint32_t>(D);
+        Dhi = static_cast<uint32_t>(D >> 32);
       }
+      // second bits set, and those whose first bit is set too
+      const uint32_t l0 = Dlo & 0x55555555u, l1 = Dhi & 0x55555555u;
+      const uint32_t n3 = __popc(l0 & (Dlo >> 1)) + __popc(l1 & (Dhi >> 1));
+      c13[i] = (__popc(l0) + __popc(l1) - n3) | (n3 << 16);
+      run += __popc(a);
     }
     const uint32_t li = w / kQuadWordsPerLine, wi = w - li * kQuadWordsPerLine;
     uint32_t* dst = s_lines + li * 32 + 4 + 2 * wi;
-    dst[0] = static_cast<uint32_t>(D);
-    dst[1] = static_cast<uint32_t>(D >> 32);
+    dst[0] = Dlo;
+    dst[1] = Dhi;
   }
-  // headers: the counts of digits 0, 1, 2 before the line's first position
-  if (tid < nl) {
-    const uint64_t P = (line0 + tid) * kQuadDigits;
-    uint64_t c0, c1, c2;
-    if (P >= n) {
-      c0 = cd(qp.nodes, 0);
-      c1 = cd(qp.nodes, 1);
-      c2 = cd(qp.nodes, 2);
-    } else {
-      const uint64_t N = quad_node_from(qp.S, qp.nodes, node0, P);
-      const uint64_t SN = detail::gld(qp.S, N);
-      const uint64_t o = rank0 + s_wrank[tid * kQuadWordsPerLine] - (cd(N, 2) + cd(N, 3));
-      const uint64_t z = (P - SN) - o;
-      const uint64_t cnt1 = cd(N + 1, 1) - cd(N, 1);
-      const uint64_t ZN = (cd(N + 1, 0) - cd(N, 0)) + cnt1;
-      const uint64_t rB = cd(N, 1) + cd(N, 3);  // ones of level 2q + 1 before S_N
-      const uint64_t d1 = detail::level_rank<1>(qp.b, SN + z) - rB;
-      const uint64_t d3 = detail::level_rank<1>(qp.b, SN + ZN + o) - (rB + cnt1);
-      c0 = cd(N, 0) + (z - d1);
-      c1 = cd(N, 1) + d1;
-      c2 = cd(N, 2) + (o - d3);
+  // headers: the counts of digits 0, 1, 2 before the line's first position,
+  // by the thread that holds the line's first word (16-bit fields: the range
+  // has 28672 positions)
+  const uint32_t mine = c13[0] + c13[1] + c13[2] + c13[3];
+  const uint32_t incl13 = detail::wave_incl_scan_u32(mine);
+  if (lane == 63) s_wave13[wave] = incl13;
+  __syncthreads();
+  uint32_t run13 = incl13 - mine;
+  for (uint32_t w = 0; w < wave; ++w) run13 += s_wave13[w];
+  run = run0;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t w = 4 * tid + i, li = w / kQuadWordsPerLine;
+    if (w < nwords && w == li * kQuadWordsPerLine) {
+      const uint32_t d1 = run13 & 0xFFFFu, d3 = run13 >> 16;
+      const uint64_t c0 = s_info[6] + (32 * w - run - d1), c1 = s_info[7] + d1,
+                     c2 = s_info[8] + (run - d3);
+      uint32_t* h = s_lines + li * 32;
+      const uint64_t h0 = c0 | (c1 << 40);
+      const uint64_t h1 = (c1 >> 24) | (c2 << 16);
+      h[0] = static_cast<uint32_t>(h0);
+      h[1] = static_cast<uint32_t>(h0 >> 32);
+      h[2] = static_cast<uint32_t>(h1);
+      h[3] = static_cast<uint32_t>(h1 >> 32);
     }
-    uint32_t* h = s_lines + tid * 32;
-    const uint64_t h0 = c0 | (c1 << 40);
-    const uint64_t h1 = (c1 >> 24) | (c2 << 16);
-    h[0] = static_cast<uint32_t>(h0);
-    h[1] = static_cast<uint32_t>(h0 >> 32);
-    h[2] = static_cast<uint32_t>(h1);
-    h[3] = static_cast<uint32_t>(h1 >> 32);
+    run13 += c13[i];
+    run += __popc(a4[i]);
   }
   __syncthreads();
   uint4* out = qp.out + line0 * 8;
@@ -1045,20 +1058,33 @@ __global__ __launch_bounds__(256) void quad_lines_kernel(QuadBuildParams qp) {
 
 // Per build workgroup g (positions from P = 448 * 64 g): the ones of level
 // 2q before P, the node N holding P (the last position when P >= n), N's
-// start and end, the ones of level 2q before N and the zeros in N -- the
-// chain of dependent loads (directory rank, node search, tables) that would
+// start and end, the ones of level 2q before N and the zeros in N, and the
+// digits 0, 1 and 2 before P -- the chain of dependent loads (directory rank, node search, tables) that would
 // otherwise hold up every build workgroup, here one thread each, all at once.
 __device__ __forceinline__ void quad_wg_one(const QuadBuildParams& qp, uint64_t g) {
   const uint64_t P = g * kQuadLinesPerWg * kQuadDigits;
   const uint64_t N = quad_node(qp.S, qp.nodes, P < qp.n ? P : qp.n - 1);
   auto cd = [&](uint64_t M, uint32_t d) { return detail::gld(qp.CD, 4 * M + d); };
   uint64_t* o = qp.wg_info + g * kQuadWgInfo;
-  o[0] = detail::level_rank<1>(qp.a, P);
+  const uint64_t r = detail::level_rank<1>(qp.a, P), SN = detail::gld(qp.S, N);
+  const uint64_t n1 = cd(N + 1, 1) - cd(N, 1), ZN = (cd(N + 1, 0) - cd(N, 0)) + n1;
+  const uint64_t OB = cd(N, 2) + cd(N, 3);
+  o[0] = r;
   o[1] = N;
-  o[2] = detail::gld(qp.S, N);
+  o[2] = SN;
   o[3] = detail::gld(qp.S, N + 1);
-  o[4] = cd(N, 2) + cd(N, 3);
-  o[5] = (cd(N + 1, 0) - cd(N, 0)) + (cd(N + 1, 1) - cd(N, 1));
+  o[4] = OB;
+  o[5] = ZN;
+  // digits 0, 1, 2 before P: the node's before it (CD), plus its digits 1
+  // and 3 up to P (the ones of level 2q + 1 in its two runs) and the rest of
+  // its zeros and ones up to P
+  const uint64_t ones = r - OB, zeros = (P - SN) - ones;
+  const uint64_t rB = cd(N, 1) + cd(N, 3);  // ones of level 2q + 1 before S_N
+  const uint64_t d1 = detail::level_rank<1>(qp.b, SN + zeros) - rB;
+  const uint64_t d3 = detail::level_rank<1>(qp.b, SN + ZN + ones) - (rB + n1);
+  o[6] = cd(N, 0) + (zeros - d1);
+  o[7] = cd(N, 1) + d1;
+  o[8] = cd(N, 2) + (ones - d3);
 }
 __global__ __launch_bounds__(256) void quad_wg_kernel(QuadBuildParams qp, uint64_t nwg) {
   const uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1412,6 +1438,51 @@ __device__ __forceinline__ void hex_lane(const HexBuildParams& hp, uint64_t t) {
                  static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32));
 }
 
+// Deposit table for 4 positions with first digits p (2 bits each): per
+// position (x, a byte each) the shift 2 (4 d0_i + r_i) of its second digit
+// among the next 4 of each run (r_i = the earlier positions with the same
+// d0); in y the bits each run advances by (a nibble each) and, from bit 16,
+// the hex digits' high halves 4 d0_i (a nibble each)
+struct HexDeposit {
+  uint2 e[256];
+};
+constexpr HexDeposit make_hex_deposit() {
+  HexDeposit t{};
+  for (uint32_t p = 0; p < 256; ++p) {
+    uint32_t x = 0, y = 0, cnt[4] = {0, 0, 0, 0};
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t d0 = (p >> (2 * i)) & 3u;
+      x |= (2 * (4 * d0 + cnt[d0])) << (8 * i);
+      y |= (4 * d0) << (16 + 4 * i);
+      ++cnt[d0];
+    }
+    for (uint32_t d = 0; d < 4; ++d) y |= (2 * cnt[d]) << (4 * d);
+    t.e[p].x = x;
+    t.e[p].y = y;
+  }
+  return t;
+}
+__device__ constexpr HexDeposit kHexDeposit = make_hex_deposit();
+
+// v + the value of the lane that a DPP control names (0 outside the row)
+template <int Ctrl>
+__device__ __forceinline__ uint64_t dpp_add_2x32(uint64_t v) {
+  const uint32_t lo = static_cast<uint32_t>(v), hi = static_cast<uint32_t>(v >> 32);
+  const uint32_t a = lo + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(lo), Ctrl, 0xF, 0xF, false));
+  const uint32_t b = hi + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(hi), Ctrl, 0xF, 0xF, false));
+  return (static_cast<uint64_t>(b) << 32) | a;
+}
+// the sum over a 16-lane row, in its last lane
+__device__ __forceinline__ uint32_t row_sum_last(uint32_t v) {
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xF, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xF, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xF, 0xF, false));
+  v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xF, 0xF, false));
+  return v;
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;           // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int kDppShr4 = 0x114, kDppShr8 = 0x118;         // row_shr
+
 // The workgroup form: 64 hex lines (8192 positions) per workgroup, one
 // 32-position word per thread.  When the positions lie in one node N, the
 // workgroup stages the quad lines of qa holding them and, per digit d0, the
@@ -1423,67 +1494,52 @@ __device__ __forceinline__ void hex_lane(const HexBuildParams& hp, uint64_t t) {
 constexpr uint32_t kHexWgLines = 64;
 constexpr uint32_t kHexWgPos = kHexWgLines * kHexDigits;         // 8192
 constexpr uint32_t kHexQaLines = kHexWgPos / kQuadDigits + 2;   // 20
-constexpr uint32_t kHexQbLines = 32;  // the four runs need at most 26
+// the four runs need at most 26 (and a window may read one word past them)
+constexpr uint32_t kHexQbLines = 32;
 
-// exclusive scans over the workgroup (4 waves) of u64 values made of 16-bit
-// fields whose sums stay below 2^16; s_w holds 4 * J u64
-template <int J>
-__device__ __forceinline__ void wg_excl_scan_fields(uint64_t (&v)[J], uint64_t* s_w,
-                                                    uint64_t (&total)[J]) {
+// exclusive scan over the workgroup (4 waves) of u64 values made of 16-bit
+// fields whose sums stay below 2^16; s_w holds 4 u64
+__device__ __forceinline__ uint64_t wg_excl_scan_fields(uint64_t v, uint64_t* s_w,
+                                                        uint64_t& total) {
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint64_t incl[J];
+  const uint64_t incl = detail::wave_incl_scan_2x32(v);
+  if (lane == 63) s_w[wave] = incl;
+  __syncthreads();
+  uint64_t before = 0, tot = 0;
 #pragma unroll
-  for (int j = 0; j < J; ++j) incl[j] = detail::wave_incl_scan_2x32(v[j]);
-  if (lane == 63) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) s_w[J * wave + j] = incl[j];
+  for (uint32_t w = 0; w < 4; ++w) {
+    const uint64_t x = s_w[w];
+    tot += x;
+    before += w < wave ? x : 0ull;
   }
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    uint64_t before = 0, tot = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < 4; ++w) {
-      const uint64_t x = s_w[J * w + j];
-      tot += x;
-      before += w < wave ? x : 0ull;
-    }
-    total[j] = tot;
-    v[j] = before + incl[j] - v[j];
-  }
-  __syncthreads();
+  total = tot;
+  return before + incl - v;
 }
 
-// Occupancy target: 7 waves per SIMD (70 VGPRs, no spills; 8 waves spill 7
-// and are no faster, 12.0 vs 12.1 ms for both levels of n = 6e9, sigma =
-// 256; the compiler's own choice is 5 waves).
+// VALU issue bounds it (0.93 of the cycles): about 760 instructions per
+// thread of 32 positions, a third of them the deposit.  Before, each window
+// divided by 14, every workgroup computed the deposit table, 4 and 16 threads
+// counted serially, and 16 counts were scanned per word instead of per line:
+// both levels of n = 2e9, sigma = 256 3.93 -> 2.84 ms.
+// Occupancy target: 7 waves per SIMD (67 VGPRs, no spills; the compiler's own
+// choice is 5 waves).
 __device__ __forceinline__ void hex_lines_wg(const HexBuildParams& hp, uint64_t blk) {
-  __shared__ __align__(16) uint4 s_qa[kHexQaLines * 8];
-  __shared__ __align__(16) uint4 s_qb[kHexQbLines * 8];
-  __shared__ uint64_t s_w[16];
-  __shared__ uint64_t s_info[1];  // staged qb lines
-  __shared__ uint64_t s_R[4], s_rb0[4], s_hx0[16];
+  // staged quad lines: their headers, and their digit words side by side (14
+  // u64 per line), so a position's word needs no division by the line's 14
+  __shared__ __align__(16) uint4 s_qah[1], s_qbh[kHexQbLines];
+  __shared__ __align__(16) uint4 s_qa[kHexQaLines * 7];
+  __shared__ __align__(16) uint4 s_qb[kHexQbLines * 7];
+  const uint64_t* qa_word = reinterpret_cast<const uint64_t*>(s_qa);
+  const uint64_t* qb_word = reinterpret_cast<const uint64_t*>(s_qb);
+  __shared__ uint64_t s_w[64];
+  __shared__ uint32_t s_nst;  // staged qb lines
+  __shared__ uint64_t s_rb0[4], s_hx0[16];
   __shared__ uint32_t s_rl[4];
-  __shared__ uint32_t s_dlut[256];
+  __shared__ uint2 s_dlut[256];
+  __shared__ uint32_t s_ro[4];  // run d's first digit within its first staged line
   const uint32_t tid = threadIdx.x;
-  // deposit table for 4 positions with first digits p (2 bits each): per
-  // position i the index 4 d0_i + r_i of its second digit among the next 4
-  // of each run (r_i = the earlier positions with the same d0), and per run
-  // the digits the 4 positions take (3 bits each, from bit 16)
-  {
-    uint32_t e = 0, cnt[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t d0 = (tid >> (2 * i)) & 3u;
-      const uint32_t r = d0 == 0 ? cnt[0] : d0 == 1 ? cnt[1] : d0 == 2 ? cnt[2] : cnt[3];
-      e |= (4 * d0 + r) << (4 * i);
-      cnt[0] += d0 == 0;
-      cnt[1] += d0 == 1;
-      cnt[2] += d0 == 2;
-      cnt[3] += d0 == 3;
-    }
-    s_dlut[tid] = e | (cnt[0] << 16) | (cnt[1] << 19) | (cnt[2] << 22) | (cnt[3] << 25);
-  }
+  s_dlut[tid] = kHexDeposit.e[tid];
   const uint64_t L0 = blk * kHexWgLines;
   const uint64_t P0 = L0 * kHexDigits;
   const uint64_t n = hp.n;
@@ -1504,63 +1560,69 @@ __device__ __forceinline__ void hex_lines_wg(const HexBuildParams& hp, uint64_t 
   const uint64_t N = na0;
   // table entries used below, issued ahead
   const uint64_t qb_d = tid < 4 ? detail::gld(hp.qbase, 4 * N + tid) : 0ull;
-  const uint64_t chd_x = tid < 16 ? detail::gld(hp.chd, 16 * N + tid) : 0ull;
-  const uint64_t qcd_x = tid < 16 ? detail::gld(hp.qcd, 4 * (4 * N + (tid >> 2)) + (tid & 3)) : 0ull;
+  uint64_t chd_x = 0, qcd_x = 0;  // of hex digit tid / 16, in its row's last lane
+  if ((tid & 15) == 15) {
+    chd_x = detail::gld(hp.chd, 16 * N + (tid >> 4));
+    qcd_x = detail::gld(hp.qcd, 16 * N + (tid >> 4));
+  }
   // ---- stage the quad lines of qa holding [P0, E)
   const uint64_t a0 = __umul64hi(P0 >> 6, 0x2492492492492493ull);
   const uint64_t a1 = __umul64hi((E - 1) >> 6, 0x2492492492492493ull);
   const uint32_t na = static_cast<uint32_t>(a1 - a0 + 1);
-  for (uint32_t i = tid; i < na * 8; i += blockDim.x) s_qa[i] = detail::gld(hp.qa, a0 * 8 + i);
+  for (uint32_t i = tid; i < na * 8; i += blockDim.x) {
+    const uint4 x = detail::gld(hp.qa, a0 * 8 + i);
+    if ((i & 7) != 0) s_qa[i - (i >> 3) - 1] = x;
+    else if (i == 0) s_qah[0] = x;
+  }
   __syncthreads();
   // ---- this thread's word and its digit counts (4 x 16-bit fields)
   const uint64_t P = P0 + 32ull * tid;
   const uint32_t valid = P < E ? (E - P < 32 ? static_cast<uint32_t>(E - P) : 32u) : 0u;
   uint64_t w = 0;
   if (valid) {
-    const uint64_t qi = __umul64hi(P >> 6, 0x2492492492492493ull);
-    w = qs_digit_word(s_qa, static_cast<uint32_t>(qi - a0),
-                      static_cast<uint32_t>(P - qi * kQuadDigits) >> 5);
+    w = qa_word[(static_cast<uint32_t>(P0 - a0 * kQuadDigits) >> 5) + tid];
   }
   const uint64_t vm = (valid == 32 ? ~0ull : (1ull << (2 * valid)) - 1) & 0x5555555555555555ull;
-  uint64_t pre[1], ctot[1];
+  uint64_t cword, ctot;
   {
     const uint64_t lo = w & vm, hi = (w >> 1) & vm;
-    pre[0] = static_cast<uint64_t>(__popcll(~(lo | hi) & vm)) |
+    cword = static_cast<uint64_t>(__popcll(~(lo | hi) & vm)) |
              (static_cast<uint64_t>(__popcll(lo & ~hi)) << 16) |
              (static_cast<uint64_t>(__popcll(hi & ~lo)) << 32) |
              (static_cast<uint64_t>(__popcll(lo & hi)) << 48);
   }
-  const uint64_t cword = pre[0];           // the word's own d's
-  wg_excl_scan_fields<1>(pre, s_w, ctot);  // pre: the d's in [P0, P)
-  // ---- the d's before P0 and the runs R_d of qb (threads 0..3)
-  if (tid < 4) {
-    const uint32_t d = tid;
-    const uint4 h = s_qa[0];
+  const uint64_t pre = wg_excl_scan_fields(cword, s_w, ctot);  // the d's in [P0, P)
+  // ---- the d's before P0 and the runs R_d of qb (wave 0: lane 16 d + k
+  // counts in word k of the first staged line, and the row's last lane sums)
+  if (tid < 64) {
+    const uint32_t d = tid >> 4, k = tid & 15;
+    const uint32_t kw = static_cast<uint32_t>(P0 - a0 * kQuadDigits) >> 5;  // < 14
+    uint32_t c = k < kw ? static_cast<uint32_t>(__popcll(quad_match(qa_word[k], d))) : 0u;
+    c = row_sum_last(c);
+    const uint4 h = s_qah[0];
     const uint64_t h0 = (uint64_t)h.x | ((uint64_t)h.y << 32);
     const uint64_t h1 = (uint64_t)h.z | ((uint64_t)h.w << 32);
     const uint64_t m40 = (1ull << 40) - 1;
     const uint64_t c0 = h0 & m40, c1 = (h0 >> 40) | ((h1 & 0xFFFFull) << 24), c2 = (h1 >> 16) & m40;
-    uint64_t g = d == 0 ? c0 : d == 1 ? c1 : d == 2 ? c2 : a0 * kQuadDigits - c0 - c1 - c2;
-    const uint32_t kw = static_cast<uint32_t>(P0 - a0 * kQuadDigits) >> 5;
-    for (uint32_t k = 0; k < kw; ++k) g += static_cast<uint64_t>(__popcll(quad_match(qs_digit_word(s_qa, 0, k), d)));
-    s_R[d] = qb_d + g;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t at = 0;
-    for (uint32_t d = 0; d < 4; ++d) {
-      const uint64_t R = s_R[d], C = (ctot[0] >> (16 * d)) & 0xFFFFull;
-      const uint64_t b0 = __umul64hi(R >> 6, 0x2492492492492493ull);
-      uint64_t b1 = __umul64hi((R + C + 31) >> 6, 0x2492492492492493ull);
-      if (b1 > hp.nql - 1) b1 = hp.nql - 1;
+    const uint64_t g = d == 0 ? c0 : d == 1 ? c1 : d == 2 ? c2 : a0 * kQuadDigits - c0 - c1 - c2;
+    const uint64_t R = __shfl(qb_d, d, 64) + g + c;  // (lane d holds digit d's base)
+    // the staged lines of run d: [b0, b1]
+    const uint64_t C = (ctot >> (16 * d)) & 0xFFFFull;
+    const uint64_t b0 = __umul64hi(R >> 6, 0x2492492492492493ull);
+    uint64_t b1 = __umul64hi((R + C + 31) >> 6, 0x2492492492492493ull);
+    if (b1 > hp.nql - 1) b1 = hp.nql - 1;
+    const uint32_t len = static_cast<uint32_t>(b1 - b0 + 1);
+    const uint32_t l0 = __shfl(len, 15, 64), l1 = __shfl(len, 31, 64), l2 = __shfl(len, 47, 64),
+                   l3 = __shfl(len, 63, 64);
+    if (k == 15) {
       s_rb0[d] = b0;
-      s_rl[d] = at;
-      at += static_cast<uint32_t>(b1 - b0 + 1);
+      s_ro[d] = static_cast<uint32_t>(R - b0 * kQuadDigits);
+      s_rl[d] = d == 0 ? 0u : d == 1 ? l0 : d == 2 ? l0 + l1 : l0 + l1 + l2;
+      if (d == 3) s_nst = l0 + l1 + l2 + l3;
     }
-    s_info[0] = at;
   }
   __syncthreads();
-  const uint32_t nst = static_cast<uint32_t>(s_info[0]);
+  const uint32_t nst = s_nst;
   if (nst > kHexQbLines) {  // not reached (at most 26); the whole workgroup
     hex_lane(hp, blk * blockDim.x + tid);
     return;
@@ -1568,39 +1630,40 @@ __device__ __forceinline__ void hex_lines_wg(const HexBuildParams& hp, uint64_t 
   for (uint32_t i = tid; i < nst * 8; i += blockDim.x) {
     const uint32_t li = i >> 3;
     const uint32_t d = li >= s_rl[3] ? 3u : li >= s_rl[2] ? 2u : li >= s_rl[1] ? 1u : 0u;
-    s_qb[i] = detail::gld(hp.qb, (s_rb0[d] + (li - s_rl[d])) * 8 + (i & 7));
+    const uint4 x = detail::gld(hp.qb, (s_rb0[d] + (li - s_rl[d])) * 8 + (i & 7));
+    if ((i & 7) != 0) s_qb[i - li - 1] = x;
+    else s_qbh[li] = x;
   }
   __syncthreads();
-  // ---- hex digits 4 x + d1 before P0 (threads 0..15): the d1's of qb before R_d0
-  if (tid < 16) {
-    const uint32_t d0 = tid >> 2, d1 = tid & 3;
-    const uint64_t R = s_R[d0], b0 = s_rb0[d0];
-    const uint32_t li = s_rl[d0];
-    const uint4 h = s_qb[li * 8];
-    const uint64_t h0 = (uint64_t)h.x | ((uint64_t)h.y << 32);
-    const uint64_t h1 = (uint64_t)h.z | ((uint64_t)h.w << 32);
-    const uint64_t m40 = (1ull << 40) - 1;
-    const uint64_t c0 = h0 & m40, c1 = (h0 >> 40) | ((h1 & 0xFFFFull) << 24), c2 = (h1 >> 16) & m40;
-    uint64_t g = d1 == 0 ? c0 : d1 == 1 ? c1 : d1 == 2 ? c2 : b0 * kQuadDigits - c0 - c1 - c2;
-    const uint32_t o = static_cast<uint32_t>(R - b0 * kQuadDigits);
-    const uint32_t kw = o >> 5, sh = 2 * (o & 31);
-    for (uint32_t k = 0; k < kw; ++k) g += static_cast<uint64_t>(__popcll(quad_match(qs_digit_word(s_qb, li, k), d1)));
-    if (sh) g += static_cast<uint64_t>(__popcll(quad_match(qs_digit_word(s_qb, li, kw), d1) & (~0ull >> (64 - sh))));
-    s_hx0[tid] = chd_x + g - qcd_x;
+  // ---- hex digits 4 d0 + d1 before P0: the d1's of qb before R_d0 (thread 16
+  // (4 d0 + d1) + k counts in word k of the run's first line)
+  {
+    const uint32_t x = tid >> 4, d0 = x >> 2, d1 = x & 3, k = tid & 15;
+    const uint32_t o = s_ro[d0], kw = o >> 5, sh = 2 * (o & 31), li = s_rl[d0];  // kw < 14
+    const uint64_t m = k < kw ? ~0ull : k == kw && sh != 0 ? ~0ull >> (64 - sh) : 0ull;
+    uint32_t c = k < 14
+                     ? static_cast<uint32_t>(__popcll(quad_match(qb_word[li * 14 + k], d1) & m))
+                     : 0u;
+    c = row_sum_last(c);
+    if (k == 15) {
+      const uint4 h = s_qbh[li];
+      const uint64_t h0 = (uint64_t)h.x | ((uint64_t)h.y << 32);
+      const uint64_t h1 = (uint64_t)h.z | ((uint64_t)h.w << 32);
+      const uint64_t m40 = (1ull << 40) - 1;
+      const uint64_t c0 = h0 & m40, c1 = (h0 >> 40) | ((h1 & 0xFFFFull) << 24), c2 = (h1 >> 16) & m40;
+      const uint64_t g = d1 == 0 ? c0 : d1 == 1 ? c1 : d1 == 2 ? c2 : s_rb0[d0] * kQuadDigits - c0 - c1 - c2;
+      s_hx0[x] = chd_x + g + c - qcd_x;
+    }
   }
   __syncthreads();
   // ---- the word's 32 hex digits: its d0's take the next digits of run d0
   auto window = [&](uint32_t d) -> uint64_t {
-    const uint64_t x = s_R[d] + ((pre[0] >> (16 * d)) & 0xFFFFull);
-    const uint64_t xl = __umul64hi(x >> 6, 0x2492492492492493ull);
-    const uint32_t o = static_cast<uint32_t>(x - xl * kQuadDigits);
-    const uint32_t k = o >> 5, sh = 2 * (o & 31);
-    const uint32_t li = s_rl[d] + static_cast<uint32_t>(xl - s_rb0[d]);
-    const uint64_t a = qs_digit_word(s_qb, li, k);
-    if (sh == 0) return a;
-    // the next word (staged whenever one of its digits is used)
-    const uint64_t b = k < 13 ? qs_digit_word(s_qb, li, k + 1) : qs_digit_word(s_qb, li + 1, 0);
-    return (a >> sh) | (b << (64 - sh));
+    const uint32_t x = s_ro[d] + (static_cast<uint32_t>(pre >> (16 * d)) & 0xFFFFu);
+    const uint32_t sh = 2 * (x & 31);
+    const uint64_t* at = qb_word + s_rl[d] * 14 + (x >> 5);
+    // (the next word is staged whenever one of its digits is used)
+    const uint64_t a = at[0], b = at[1];
+    return (a >> sh) | ((b << 1) << (63 - sh));
   };
   const uint64_t W[4] = {window(0), window(1), window(2), window(3)};
   // 4 positions at a time: the next 4 digits of each window side by side in
@@ -1612,48 +1675,60 @@ __device__ __forceinline__ void hex_lines_wg(const HexBuildParams& hp, uint64_t 
     uint64_t S0 = W[0], S1 = W[1], S2 = W[2], S3 = W[3];
 #pragma unroll
     for (uint32_t c = 0; c < 8; ++c) {
-      const uint32_t L = s_dlut[static_cast<uint32_t>(w >> (8 * c)) & 0xFFu];
+      const uint2 L = s_dlut[static_cast<uint32_t>(w >> (8 * c)) & 0xFFu];
       const uint32_t C = (static_cast<uint32_t>(S0) & 0xFFu) | ((static_cast<uint32_t>(S1) & 0xFFu) << 8) |
                          ((static_cast<uint32_t>(S2) & 0xFFu) << 16) |
-                         ((static_cast<uint32_t>(S3) & 0xFFu) << 24);
-      uint32_t out = 0;
+                         (static_cast<uint32_t>(S3) << 24);
+      uint32_t out = L.y >> 16;
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t idx = (L >> (4 * i)) & 15u;
-        out |= ((idx & 12u) | ((C >> (2 * idx)) & 3u)) << (4 * i);
-      }
-      S0 >>= 2 * ((L >> 16) & 7u);
-      S1 >>= 2 * ((L >> 19) & 7u);
-      S2 >>= 2 * ((L >> 22) & 7u);
-      S3 >>= 2 * ((L >> 25) & 7u);
+      for (uint32_t i = 0; i < 4; ++i) out |= ((C >> ((L.x >> (8 * i)) & 31u)) & 3u) << (4 * i);
+      S0 >>= L.y & 15u;
+      S1 >>= (L.y >> 4) & 15u;
+      S2 >>= (L.y >> 8) & 15u;
+      S3 >>= (L.y >> 12) & 15u;
       if (c < 4) lo |= static_cast<uint64_t>(out) << (16 * c);
       else hi |= static_cast<uint64_t>(out) << (16 * (c - 4));
     }
     lo &= valid >= 16 ? ~0ull : (1ull << (4 * valid)) - 1;
     hi &= valid >= 32 ? ~0ull : valid > 16 ? (1ull << (4 * (valid - 16))) - 1 : 0ull;
   }
-  // ---- the word's hex-digit counts (field d1 of hh[d0]): the d1's among the
-  // digits its d0's used from window d0; scanned
-  uint64_t hh[4], htot[4];
+  // ---- the counts of hex digits 4q .. 4q + 3 (16-bit fields) in line l =
+  // tid / 4, by its lane q = tid % 4: per word the d1's among the digits its
+  // d0's used from window d0, added up over the line's four words
+  const uint64_t l = L0 + (tid >> 2);
+  const uint32_t q = tid & 3;
+  uint64_t line_cnt = 0;
 #pragma unroll
   for (uint32_t d0 = 0; d0 < 4; ++d0) {
     const uint32_t c = static_cast<uint32_t>(cword >> (16 * d0)) & 0xFFFFu;  // <= 32
-    const uint64_t m = c >= 32 ? ~0ull : (1ull << (2 * c)) - 1;
-    uint64_t f = 0;
-#pragma unroll
-    for (uint32_t d1 = 0; d1 < 4; ++d1)
-      f |= static_cast<uint64_t>(__popcll(quad_match(W[d0], d1) & m)) << (16 * d1);
-    hh[d0] = f;
+    const uint64_t m = (c >= 32 ? ~0ull : (1ull << (2 * c)) - 1) & 0x5555555555555555ull;
+    const uint64_t lo = W[d0] & m, hi = (W[d0] >> 1) & m;
+    const uint32_t nlo = __popcll(lo), nhi = __popcll(hi), n3 = __popcll(lo & hi);
+    uint64_t f = static_cast<uint64_t>((c - nlo - nhi + n3) | ((nlo - n3) << 16)) |
+                 (static_cast<uint64_t>((nhi - n3) | (n3 << 16)) << 32);
+    f = dpp_add_2x32<kDppXor2>(dpp_add_2x32<kDppXor1>(f));
+    line_cnt = q == d0 ? f : line_cnt;
   }
-  wg_excl_scan_fields<4>(hh, s_w, htot);  // hh: the hex digits in [P0, P)
+  // the counts before each line: inclusive over the 4 lines of a 16-lane row,
+  // then over the workgroup's 16 rows, whose sums every wave scans with one
+  // lane per (row, q)
+  const uint64_t row_incl = dpp_add_2x32<kDppShr8>(dpp_add_2x32<kDppShr4>(line_cnt));
+  if ((tid & 15) >= 12) s_w[(tid >> 4) * 4 + q] = row_incl;
+  __syncthreads();
+  uint64_t mine;
+  {
+    const uint64_t x = s_w[tid & 63];
+    uint64_t incl = dpp_add_2x32<kDppShr8>(dpp_add_2x32<kDppShr4>(x));
+    const uint32_t lane = tid & 63;
+    // lane 16 g + 12 + q holds group g's sum of q; the groups before lane's
+    const uint64_t g0 = __shfl(incl, 12 + q, 64), g1 = __shfl(incl, 28 + q, 64),
+                   g2 = __shfl(incl, 44 + q, 64);
+    incl += lane >= 48 ? g0 + g1 + g2 : lane >= 32 ? g0 + g1 : lane >= 16 ? g0 : 0ull;
+    const uint64_t before = __shfl(incl - x, (tid >> 4) * 4 + q, 64);
+    mine = before + row_incl - line_cnt;
+  }
   // ---- write: the digits, and the counts of hex digits 4q .. 4q + 3 before
-  // the line (its first word's prefix, from lane 4 (tid / 4))
-  const uint64_t l = L0 + (tid >> 2);
-  const uint32_t q = tid & 3;
-  const uint32_t src = (tid & 63u) & ~3u;
-  const uint64_t f0 = __shfl(hh[0], src, 64), f1 = __shfl(hh[1], src, 64),
-                 f2 = __shfl(hh[2], src, 64), f3 = __shfl(hh[3], src, 64);
-  const uint64_t mine = q == 0 ? f0 : q == 1 ? f1 : q == 2 ? f2 : f3;
+  // the line
   if (l < hp.nlines) {
     hp.out[l * 8 + (q < 2 ? 2 + q : 4 + q)] =
         make_uint4(static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
