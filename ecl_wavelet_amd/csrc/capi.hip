@@ -479,6 +479,120 @@ uint64_t available_host_memory() {
 static hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 // ===========================================================================
+// host-issued batches
+// ===========================================================================
+// A pipe is what one host-issued batch call works with: kPipeSlots
+// default-priority streams, each with pinned input and output buffers grown
+// on demand.  Calls take an idle pipe of their device (or make one) and put
+// it back, so a tree's first call does not pay for streams and pinned memory
+// (about 0.45 ms to make and unmake for a tree that is asked three times),
+// and calls from several threads, on one tree or many, have a pipe each.  At
+// most kIdlePipes wait per device; ecl_release_cached_memory gives them back.
+namespace ecl {
+namespace lib {
+namespace {
+constexpr int kPipeSlots = 3;
+constexpr size_t kIdlePipes = 4;
+constexpr size_t kPipeMinBytes = size_t(1) << 20;  // smallest buffer of a slot
+constexpr int kPipeDevices = 64;
+
+struct HostPipe {
+  int device = 0;
+  hipStream_t stream[kPipeSlots] = {};
+  void* pin_in[kPipeSlots] = {};
+  void* pin_out[kPipeSlots] = {};
+  size_t cap_in[kPipeSlots] = {}, cap_out[kPipeSlots] = {};
+  ~HostPipe() {
+    for (int i = 0; i < kPipeSlots; ++i) {
+      if (stream[i]) (void)hipStreamDestroy(stream[i]);
+      if (pin_in[i]) (void)hipHostFree(pin_in[i]);
+      if (pin_out[i]) (void)hipHostFree(pin_out[i]);
+    }
+  }
+  static void grow(void*& pin, size_t& cap, size_t bytes) {
+    if (bytes <= cap) return;
+    if (pin) ECL_HIP(hipHostFree(pin));
+    pin = nullptr;
+    cap = 0;
+    bytes = std::max(bytes, kPipeMinBytes);
+    ECL_HIP(hipHostMalloc(&pin, bytes, hipHostMallocDefault));
+    cap = bytes;
+  }
+  void reserve(int slots, size_t in_bytes, size_t out_bytes) {
+    for (int i = 0; i < slots; ++i) {
+      if (!stream[i]) ECL_HIP(hipStreamCreate(&stream[i]));
+      grow(pin_in[i], cap_in[i], in_bytes);
+      grow(pin_out[i], cap_out[i], out_bytes);
+    }
+  }
+};
+
+struct PipePool {
+  std::mutex mu;
+  std::vector<std::unique_ptr<HostPipe>> idle;
+};
+// never destroyed: see g_pool
+PipePool* const g_pipes = new PipePool[kPipeDevices];
+
+// a pipe of the device for the length of one call; one whose call failed is
+// not handed on
+class PipeLease {
+ public:
+  explicit PipeLease(int device) {
+    if (device >= 0 && device < kPipeDevices) {
+      PipePool& P = g_pipes[device];
+      std::lock_guard<std::mutex> lk(P.mu);
+      if (!P.idle.empty()) {
+        pipe_ = std::move(P.idle.back());
+        P.idle.pop_back();
+      }
+    }
+    if (!pipe_) pipe_.reset(new HostPipe());
+    pipe_->device = device;
+  }
+  ~PipeLease() {
+    if (!done_) {  // its kernels may still run
+      for (hipStream_t st : pipe_->stream)
+        if (st) (void)hipStreamSynchronize(st);
+      (void)hipGetLastError();
+      return;
+    }
+    const int device = pipe_->device;
+    if (device < 0 || device >= kPipeDevices) return;
+    PipePool& P = g_pipes[device];
+    std::unique_lock<std::mutex> lk(P.mu);
+    if (P.idle.size() < kIdlePipes) {
+      P.idle.push_back(std::move(pipe_));
+    } else {
+      lk.unlock();
+      pipe_.reset();
+    }
+  }
+  PipeLease(const PipeLease&) = delete;
+  PipeLease& operator=(const PipeLease&) = delete;
+  HostPipe* operator->() const { return pipe_.get(); }
+  void done() { done_ = true; }  // every stream of the pipe is idle
+
+ private:
+  std::unique_ptr<HostPipe> pipe_;
+  bool done_ = false;
+};
+}  // namespace
+
+void release_host_pipes(int device) {
+  if (device < 0 || device >= kPipeDevices) return;
+  std::vector<std::unique_ptr<HostPipe>> gone;
+  {
+    std::lock_guard<std::mutex> lk(g_pipes[device].mu);
+    gone.swap(g_pipes[device].idle);
+  }
+  DeviceScope ds(device);
+  gone.clear();
+}
+}  // namespace lib
+}  // namespace ecl
+
+// ===========================================================================
 // objects
 // ===========================================================================
 struct ecl_bit_array_t {
@@ -501,46 +615,6 @@ struct ecl_rank_select_t {
   std::vector<LevelView> levels;
   uint64_t total_l2 = 0;
   ~ecl_rank_select_t() { delete ba; }
-};
-
-// Host-issued batches: two default-priority streams, pinned staging and
-// device buffers per stream, grown on demand and kept with the handle.
-struct HostPipe {
-  hipStream_t stream[2] = {nullptr, nullptr};
-  void* pin_in[2] = {nullptr, nullptr};
-  void* pin_out[2] = {nullptr, nullptr};
-  DevBuf d_in[2], d_out[2];
-  size_t cap_in = 0, cap_out = 0;
-  std::mutex mu;
-  ~HostPipe() {
-    for (int i = 0; i < 2; ++i) {
-      if (stream[i]) (void)hipStreamDestroy(stream[i]);
-      if (pin_in[i]) (void)hipHostFree(pin_in[i]);
-      if (pin_out[i]) (void)hipHostFree(pin_out[i]);
-    }
-  }
-  void reserve(size_t in_bytes, size_t out_bytes) {
-    for (int i = 0; i < 2; ++i)
-      if (!stream[i]) ECL_HIP(hipStreamCreate(&stream[i]));
-    if (in_bytes > cap_in) {
-      for (int i = 0; i < 2; ++i) {
-        if (pin_in[i]) ECL_HIP(hipHostFree(pin_in[i]));
-        pin_in[i] = nullptr;
-        ECL_HIP(hipHostMalloc(&pin_in[i], in_bytes, hipHostMallocDefault));
-        d_in[i] = DevBuf(in_bytes);
-      }
-      cap_in = in_bytes;
-    }
-    if (out_bytes > cap_out) {
-      for (int i = 0; i < 2; ++i) {
-        if (pin_out[i]) ECL_HIP(hipHostFree(pin_out[i]));
-        pin_out[i] = nullptr;
-        ECL_HIP(hipHostMalloc(&pin_out[i], out_bytes, hipHostMallocDefault));
-        d_out[i] = DevBuf(out_bytes);
-      }
-      cap_out = out_bytes;
-    }
-  }
 };
 
 struct ecl_wavelet_tree_t {
@@ -569,7 +643,6 @@ struct ecl_wavelet_tree_t {
   DevBuf hex_lines, hex_tab;                // optional hex lines, bases and superblocks
   HexView hex{};
   DevBuf d_layouts;  // device copies of quad and hex (once asked for; kept current)
-  std::unique_ptr<HostPipe> pipe{new HostPipe()};
   ~ecl_wavelet_tree_t() { delete rs; }
 };
 
@@ -2175,6 +2248,7 @@ ecl_status ecl_release_cached_memory(int device) {
   return guard([&] {
     set_device(device);
     release_scratch_cache(device);
+    release_host_pipes(device);
     release_block_pool(device);
   });
 }
@@ -2672,44 +2746,105 @@ size_t ecl_wavelet_tree_needed_gpu_memory(size_t n, size_t sigma, uint8_t L, siz
   return tree_needed_bytes(n, sigma, L, 8, false);
 }
 
-// Chunked host batch (the reference's graph of H2D -> kernel -> D2H per
-// chunk, wavelet_tree.cuh:94-151, 1121-1211): chunk i uses stream i % 2; the
-// host copies chunk i+1 into pinned memory while chunk i runs, and copies
-// the results of chunk i-2 out before reusing its buffers.
 }  // extern "C"
+
+// A host batch, in chunks of at most kPipeChunk queries, chunk c in slot c %
+// kPipeSlots (after the reference's graph of H2D -> kernel -> D2H per chunk,
+// wavelet_tree.cuh:94-151, 1121-1211).  There are no transfers of their own:
+// the kernels read the queries from pinned memory and write the results to
+// pinned memory over the host link, so the bytes move while other waves wait
+// for their lines.  With copy commands around the kernels the three ran one
+// after the other, whatever their streams (n = 2^30, sigma = 64, 10^7
+// queries: access 4.26, rank 7.4, select 9.0 ms; now 2.3, 3.7 and 4.75 ms,
+// where the queries alone take 1.4, 2.8 and 2.8 ms of the link).  Three
+// slots of 2^19 queries: with two access took 3.1 ms, with four 2.65; chunks
+// of 2^18 took 2.95, of 2^20 and 2^21 the same.  A batch of up to kPipeSlots
+// chunks is queued and then collected by the calling thread; of a longer one
+// a second thread collects the results, in order.
+constexpr size_t kPipeChunk = size_t(1) << 19;
 
 template <typename Launch>
 static void pipelined(ecl_wavelet_tree wt, const void* in, size_t in_elem, void* out,
                       size_t out_elem, size_t m, const char* kind, Launch&& launch) {
-  HostPipe& P = *wt->pipe;
-  std::lock_guard<std::mutex> lk(P.mu);
-  const size_t chunk = std::min<size_t>(m, kHostChunk / 4);
+  const size_t chunk = std::min(m, kPipeChunk);
   const size_t nchunks = (m + chunk - 1) / chunk;
-  check_query_memory(2 * chunk * (in_elem + out_elem), kind);
-  P.reserve(chunk * in_elem, chunk * out_elem);
-  size_t pending_off[2] = {0, 0}, pending_len[2] = {0, 0};
-  auto drain = [&](int b) {
-    if (!pending_len[b]) return;
-    ECL_HIP(hipStreamSynchronize(P.stream[b]));
-    parallel_memcpy(static_cast<uint8_t*>(out) + pending_off[b] * out_elem, P.pin_out[b],
-                    pending_len[b] * out_elem);
-    pending_len[b] = 0;
-  };
-  for (size_t c = 0; c < nchunks; ++c) {
-    const int b = static_cast<int>(c & 1);
+  // admission as for two staging chunks of kHostChunk / 4 on the device; a
+  // batch of one chunk asks while its kernel runs
+  const uint64_t need = 2 * std::min<uint64_t>(m, kHostChunk / 4) * (in_elem + out_elem);
+  if (nchunks > 1) check_query_memory(need, kind);
+  PipeLease P(wt->device);
+  P->reserve(static_cast<int>(std::min<size_t>(nchunks, kPipeSlots)), chunk * in_elem,
+             chunk * out_elem);
+  const auto* src = static_cast<const uint8_t*>(in);
+  auto* dst = static_cast<uint8_t*>(out);
+  auto put = [&](size_t c) {
+    const int b = static_cast<int>(c % kPipeSlots);
     const size_t off = c * chunk, len = std::min(chunk, m - off);
-    drain(b);
-    parallel_memcpy(P.pin_in[b], static_cast<const uint8_t*>(in) + off * in_elem, len * in_elem);
-    ECL_HIP(hipMemcpyAsync(P.d_in[b].ptr, P.pin_in[b], len * in_elem, hipMemcpyHostToDevice,
-                           P.stream[b]));
-    launch(P.d_in[b].ptr, len, P.d_out[b].ptr, P.stream[b]);
-    ECL_HIP(hipMemcpyAsync(P.pin_out[b], P.d_out[b].ptr, len * out_elem,
-                           hipMemcpyDeviceToHost, P.stream[b]));
-    pending_off[b] = off;
-    pending_len[b] = len;
+    parallel_memcpy(P->pin_in[b], src + off * in_elem, len * in_elem);
+    launch(P->pin_in[b], len, P->pin_out[b], P->stream[b]);
+  };
+  auto take = [&](size_t c) {
+    const int b = static_cast<int>(c % kPipeSlots);
+    const size_t off = c * chunk, len = std::min(chunk, m - off);
+    ECL_HIP(hipStreamSynchronize(P->stream[b]));
+    parallel_memcpy(dst + off * out_elem, P->pin_out[b], len * out_elem);
+  };
+  if (nchunks <= kPipeSlots) {
+    for (size_t c = 0; c < nchunks; ++c) put(c);
+    if (nchunks == 1) check_query_memory(need, kind);
+    for (size_t c = 0; c < nchunks; ++c) take(c);
+    P.done();
+    return;
   }
-  drain(0);
-  drain(1);
+  std::mutex mu;
+  std::condition_variable cv;
+  size_t queued = 0, taken = 0;
+  std::exception_ptr failed;
+  bool stop = false;
+  std::thread taker([&] {
+    try {
+      ECL_HIP(hipSetDevice(wt->device));
+      for (size_t c = 0; c < nchunks; ++c) {
+        {
+          std::unique_lock<std::mutex> lk(mu);
+          cv.wait(lk, [&] { return queued > c || stop; });
+          if (queued <= c) return;
+        }
+        take(c);
+        std::lock_guard<std::mutex> lk(mu);
+        taken = c + 1;
+        cv.notify_all();
+      }
+    } catch (...) {
+      std::lock_guard<std::mutex> lk(mu);
+      failed = std::current_exception();
+      cv.notify_all();
+    }
+  });
+  try {
+    for (size_t c = 0; c < nchunks; ++c) {
+      {
+        std::unique_lock<std::mutex> lk(mu);
+        cv.wait(lk, [&] { return c < taken + kPipeSlots || failed; });
+        if (failed) break;
+      }
+      put(c);
+      std::lock_guard<std::mutex> lk(mu);
+      queued = c + 1;
+      cv.notify_all();
+    }
+  } catch (...) {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      stop = true;
+      cv.notify_all();
+    }
+    taker.join();
+    throw;
+  }
+  taker.join();
+  if (failed) std::rethrow_exception(failed);
+  P.done();
 }
 
 extern "C" {

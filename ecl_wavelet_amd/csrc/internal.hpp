@@ -67,6 +67,8 @@ constexpr size_t kPoolMinBytes = size_t(1) << 20;
 size_t pooled_bytes(int device);
 // frees every cached block of the device
 void release_block_pool(int device);
+// frees the idle pinned buffers of the host query calls (capi.hip)
+void release_host_pipes(int device);
 
 // ---- kernel profiling (events around selected launches) -------------------
 enum KernelId : int {

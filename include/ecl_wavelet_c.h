@@ -114,11 +114,13 @@ ecl_status ecl_device_synchronize(int device);
 ecl_status ecl_device_mem_info(int device, size_t* free_bytes, size_t* total_bytes);
 /* The library keeps freed device blocks of 1 MiB or more per device and
  * hands them out again for requests of the same size class (up to 40% of
- * the device's memory; freed when an allocation would fail), and keeps the
+ * the device's memory; freed when an allocation would fail), keeps the
  * construction scratch (tile histograms and their scan, about 0.1 bytes per
- * symbol) for the next build.  This frees both.  No counterpart in the
- * reference, which allocates and frees per call; for callers that need the
- * memory back outside the library. */
+ * symbol) for the next build, and keeps up to four idle sets of the host
+ * query calls' staging buffers (each at most 36 MB of pinned host memory).
+ * This frees all three.
+ * No counterpart in the reference, which allocates and frees per call; for
+ * callers that need the memory back outside the library. */
 ecl_status ecl_release_cached_memory(int device);
 /* Caps the free device memory the library's admission checks assume on a
  * device (tree builds, query batches, server budgets): they see at most
