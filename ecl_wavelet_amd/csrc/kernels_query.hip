@@ -155,6 +155,58 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void t
 }
 
 // ---------------------------------------------------------------------------
+// Short batches over the binary levels: G lanes per query, each reading its
+// share of a level's words (the device API's group descents).  A short batch
+// leaves most of the chip idle and takes as long as one wave's descent: a
+// chain of line latencies, and in one lane the instructions between them (at
+// 1000 queries per wave slot the directory select spent 7.5 us a level).
+// With the work of a level spread over lanes, n = 5e8, sigma = 256, 1000
+// queries, directory: access 10.3 -> 9.1, rank 11.3 -> 10.3, select 60 -> 27
+// us; query and select lines: 13.5 -> 8.8, 15.3 -> 9.6, 27.5 -> 17.4 us; 2^16
+// symbols, n = 5e7: select 150 -> 51 and 108 -> 37 us.
+template <typename T, int G>
+__global__ __launch_bounds__(256) void tree_access_group_kernel(
+    TreeQueryParams p, const uint64_t* __restrict__ idx, uint64_t m, T* __restrict__ out) {
+  extern __shared__ uint8_t s_meta[];
+  const uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / G;
+  const uint64_t i = q < m ? idx[q] : ~0ull;
+  const Meta mt = stage_meta(p.view, s_meta);
+  if (i >= p.view.n) return;
+  const T* amap = static_cast<const T*>(p.alphabet_out);
+  const uint64_t r = detail::tree_access<false, G>(p.view, mt.lv, mt.counts, mt.ranks, mt.nal, i);
+  if (threadIdx.x % G == 0) out[q] = amap ? amap[r] : static_cast<T>(r);
+}
+template <typename T, int G>
+__global__ __launch_bounds__(256) void tree_rank_group_kernel(
+    TreeQueryParams p, const uint8_t* __restrict__ qs, uint64_t m, uint64_t* __restrict__ out) {
+  extern __shared__ uint8_t s_meta[];
+  const uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / G;
+  const uint8_t* e = qs + (q < m ? q : m - 1) * 16;
+  const uint64_t i = *reinterpret_cast<const uint64_t*>(e);
+  const uint64_t c = map_symbol<T>(p, load_sym(e, sizeof(T)));
+  const Meta mt = stage_meta(p.view, s_meta);
+  if (q >= m) return;
+  const uint64_t r = i > p.view.n ? 0
+                                  : detail::tree_rank<false, G>(p.view, mt.lv, mt.counts,
+                                                                mt.ranks, mt.nal, c, i);
+  if (threadIdx.x % G == 0) out[q] = r;
+}
+template <typename T, int G>
+__global__ __launch_bounds__(256) void tree_select_group_kernel(
+    TreeQueryParams p, const uint8_t* __restrict__ qs, uint64_t m, uint64_t* __restrict__ out) {
+  extern __shared__ uint8_t s_meta[];
+  const uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / G;
+  const uint8_t* e = qs + (q < m ? q : m - 1) * 16;
+  const uint64_t k = *reinterpret_cast<const uint64_t*>(e);
+  const uint64_t c = map_symbol<T>(p, load_sym(e, sizeof(T)));
+  const Meta mt = stage_meta(p.view, s_meta);
+  if (q >= m) return;
+  const uint64_t r = detail::tree_select<true, false, G>(p.view, mt.lv, mt.counts, mt.ranks,
+                                                         mt.nal, c, k);
+  if (threadIdx.x % G == 0) out[q] = r;
+}
+
+// ---------------------------------------------------------------------------
 // Access and rank over quad lines (see QuadView): one 128-byte line per two
 // levels.  Two adjacent lanes share a query: lane 0 loads the line's header
 // and digit words 0..5, lane 1 words 6..13; each counts the digit in its
@@ -942,6 +994,60 @@ void rank_hex(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t*
   }
 }
 
+// Lanes per query of a short batch over the binary levels: 16 up to 2^13
+// queries, 8 up to `max8` (0: none), then 0 (the kernels for throughput).
+// Measured on n = 5e8, sigma = 256 in us, one lane (a pair over lines), 8 and
+// 16 lanes per query.  Directory select: 8000 queries 82 / 40 / 40, 16000 75 /
+// 45 / 46, 30000 73 / 50 / 65 (one lane over hints 55, 51, 47); over select
+// lines: 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access over query lines: 15.1 / 11.5 / 10.9, 15.6 / 12 /
+// 12.8, 16.5 / 14.6 / 19.5; over the directory 8 lanes gain nothing past 2^13
+// (16000: 13.9 / 13.4 / 14.2).
+constexpr uint64_t kGroup16Max = 1u << 13, kGroup8Max = 1u << 14;
+int group_lanes(uint64_t m, uint64_t max8) {
+  return m <= kGroup16Max ? 16 : m <= max8 ? 8 : 0;
+}
+// access and rank: not when the caller has set the lanes per query
+int group_lanes(const TreeQueryParams& p, uint64_t m, uint64_t max8) {
+  return p.lanes != 0 || g_query_lanes.load() != 0 ? 0 : group_lanes(m, max8);
+}
+
+template <int G>
+void access_group(const TreeQueryParams& p, const uint64_t* idx, uint64_t m, void* out,
+                  hipStream_t s) {
+  const dim3 g(static_cast<uint32_t>((m * G + 255) / 256)), b(256);
+  const size_t sh = meta_bytes(p.view);
+  switch (p.esize) {
+    case 1: hipLaunchKernelGGL((tree_access_group_kernel<uint8_t, G>), g, b, sh, s, p, idx, m, static_cast<uint8_t*>(out)); break;
+    case 2: hipLaunchKernelGGL((tree_access_group_kernel<uint16_t, G>), g, b, sh, s, p, idx, m, static_cast<uint16_t*>(out)); break;
+    case 4: hipLaunchKernelGGL((tree_access_group_kernel<uint32_t, G>), g, b, sh, s, p, idx, m, static_cast<uint32_t*>(out)); break;
+    default: hipLaunchKernelGGL((tree_access_group_kernel<uint64_t, G>), g, b, sh, s, p, idx, m, static_cast<uint64_t*>(out)); break;
+  }
+}
+template <int G>
+void rank_group(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t* out,
+                hipStream_t s) {
+  const dim3 g(static_cast<uint32_t>((m * G + 255) / 256)), b(256);
+  const size_t sh = meta_bytes(p.view);
+  switch (p.esize) {
+    case 1: hipLaunchKernelGGL((tree_rank_group_kernel<uint8_t, G>), g, b, sh, s, p, qq, m, out); break;
+    case 2: hipLaunchKernelGGL((tree_rank_group_kernel<uint16_t, G>), g, b, sh, s, p, qq, m, out); break;
+    case 4: hipLaunchKernelGGL((tree_rank_group_kernel<uint32_t, G>), g, b, sh, s, p, qq, m, out); break;
+    default: hipLaunchKernelGGL((tree_rank_group_kernel<uint64_t, G>), g, b, sh, s, p, qq, m, out); break;
+  }
+}
+template <int G>
+void select_group(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t* out,
+                  hipStream_t s) {
+  const dim3 g(static_cast<uint32_t>((m * G + 255) / 256)), b(256);
+  const size_t sh = meta_bytes(p.view);
+  switch (p.esize) {
+    case 1: hipLaunchKernelGGL((tree_select_group_kernel<uint8_t, G>), g, b, sh, s, p, qq, m, out); break;
+    case 2: hipLaunchKernelGGL((tree_select_group_kernel<uint16_t, G>), g, b, sh, s, p, qq, m, out); break;
+    case 4: hipLaunchKernelGGL((tree_select_group_kernel<uint32_t, G>), g, b, sh, s, p, qq, m, out); break;
+    default: hipLaunchKernelGGL((tree_select_group_kernel<uint64_t, G>), g, b, sh, s, p, qq, m, out); break;
+  }
+}
+
 void launch_tree_access(const TreeQueryParams& p, const uint64_t* idx,
                         uint64_t m, void* out, hipStream_t s) {
   if (m == 0) return;
@@ -952,6 +1058,9 @@ void launch_tree_access(const TreeQueryParams& p, const uint64_t* idx,
   } else if (p.quad.levels) {
     if (p.quad.nbase <= kQuadLdsBase) access_quad<true>(p, idx, m, out, s);
     else access_quad<false>(p, idx, m, out, s);
+  } else if (const int g = group_lanes(p, m, p.has_lines ? kGroup8Max : 0)) {
+    if (g == 16) access_group<16>(p, idx, m, out, s);
+    else access_group<8>(p, idx, m, out, s);
   } else if (pair_lanes(p)) access_g<2>(p, idx, m, out, s);
   else access_g<1>(p, idx, m, out, s);
   ECL_HIP(hipGetLastError());
@@ -981,6 +1090,9 @@ void launch_tree_rank(const TreeQueryParams& p, const void* q, uint64_t m,
   } else if (p.quad.levels) {
     if (p.quad.nbase <= kQuadLdsBase) rank_quad<true>(p, qq, m, out, s);
     else rank_quad<false>(p, qq, m, out, s);
+  } else if (const int g = group_lanes(p, m, p.has_lines ? kGroup8Max : 0)) {
+    if (g == 16) rank_group<16>(p, qq, m, out, s);
+    else rank_group<8>(p, qq, m, out, s);
   } else if (pair_lanes(p)) rank_g<2>(p, qq, m, out, s);
   else rank_g<1>(p, qq, m, out, s);
   ECL_HIP(hipGetLastError());
@@ -1020,6 +1132,9 @@ void launch_tree_select(const TreeQueryParams& p, const void* q, uint64_t m,
   if (p.quad.has_sel) {
     if (p.quad.ntab <= kQuadLdsTab) select_quad<true>(p, qq, m, out, s);
     else select_quad<false>(p, qq, m, out, s);
+  } else if (const int g = group_lanes(m, p.has_sel_lines || p.has_lines ? kGroup8Max : 2 * kGroup8Max)) {
+    if (g == 16) select_group<16>(p, qq, m, out, s);
+    else select_group<8>(p, qq, m, out, s);
   } else if (p.has_sel_lines) select_sl<true>(p, qq, m, out, s);
   else select_sl<false>(p, qq, m, out, s);
   ECL_HIP(hipGetLastError());

@@ -662,36 +662,44 @@ __device__ __forceinline__ uint64_t level_rank_coop(const LevelView& v, uint64_t
   return Value ? ones : index - ones;
 }
 
-// position of the r-th (1-based) Value in the nw words from w (the first
-// word's bits below off dropped), the words split over the group in
+// position of the r-th (1-based) Value in the nw <= 15 words from w (the
+// first word's bits below off dropped), the words split over the group in
 // contiguous shares; `none` when the words hold fewer than r
 template <int Value, int G>
 __device__ __forceinline__ uint64_t group_select_words(const uint64_t* w, uint32_t nw,
                                                        uint32_t off, uint64_t r,
                                                        uint64_t pos0, uint64_t none) {
+  constexpr uint32_t W = (15 + G - 1) / G;
   const uint32_t t = group_lane<G>();
-  const uint32_t k0 = t * nw / G, k1 = (t + 1) * nw / G;
+  const uint32_t per = (nw + G - 1) / G, k0 = t * per;
+  uint64_t x[W];
   uint32_t cnt = 0;
-  for (uint32_t k = k0; k < k1; ++k) {
-    uint64_t x = Value ? gld(w, k) : ~gld(w, k);
-    if (k == 0) x &= ~0ull << off;
-    cnt += static_cast<uint32_t>(__popcll(x));
+#pragma unroll
+  for (uint32_t j = 0; j < W; ++j) {
+    const uint32_t k = k0 + j;
+    x[j] = 0;
+    if (j < per && k < nw) {
+      x[j] = Value ? gld(w, k) : ~gld(w, k);
+      if (k == 0) x[j] &= ~0ull << off;
+    }
+    cnt += static_cast<uint32_t>(__popcll(x[j]));
   }
   const uint32_t ex = group_excl_scan<G>(cnt);
   const bool own = ex < r && r <= static_cast<uint64_t>(ex) + cnt;
   uint64_t pos = none;
   if (own) {
-    uint64_t rr = r - ex;
-    for (uint32_t k = k0; k < k1; ++k) {
-      uint64_t x = Value ? gld(w, k) : ~gld(w, k);
-      if (k == 0) x &= ~0ull << off;
-      const uint32_t c = static_cast<uint32_t>(__popcll(x));
-      if (rr <= c) {
-        pos = pos0 + 64ull * k + select_in_word(x, static_cast<uint32_t>(rr));
-        break;
+    uint32_t rr = static_cast<uint32_t>(r - ex), kk = k0;
+    uint64_t y = x[0];
+#pragma unroll
+    for (uint32_t j = 0; j + 1 < W; ++j) {  // the share's word that holds it
+      const uint32_t c = static_cast<uint32_t>(__popcll(y));
+      if (kk == k0 + j && rr > c) {
+        rr -= c;
+        y = x[j + 1];
+        ++kk;
       }
-      rr -= c;
     }
+    pos = pos0 + 64ull * kk + select_in_word(y, rr);
   }
   bool any = false;
   pos = group_from<G>(own, pos, &any);
@@ -734,22 +742,30 @@ __device__ __forceinline__ uint64_t level_select_coop(const LevelView& v, uint64
     if (c < i) b_lo = mid; else b_hi = mid - 1;
   }
   const uint64_t blk1 = b_lo;
-  const uint64_t e1 = gld(v.l1, blk1);
-  const uint64_t r = i - (Value ? e1 : (blk1 << 16) - e1);
   uint64_t k_lo = lo_pos >> 9, k_hi = hi_pos >> 9;
   const uint64_t first = blk1 << 7, last = first + kL2PerL1 - 1;
   if (k_lo < first) k_lo = first;
   if (k_hi > last) k_hi = last;
   // blocks k_lo + u (0 < u <= span) with fewer than r Values before them
-  // (the counts grow with u): counted by the lanes together
-  uint32_t below = 0;
-  for (uint64_t u = 1 + group_lane<G>(); u <= k_hi - k_lo; u += G) {
+  // (the counts grow with u), counted by the lanes together.  Lane u's first
+  // entry, k_lo + u, is read beside the L1 entry, and the answer's entry
+  // comes from the lane that read it.
+  const uint64_t span = k_hi - k_lo;
+  const uint32_t t = group_lane<G>();
+  const uint64_t e0 = t <= span ? gld(v.l2, k_lo + t) : 0;
+  const uint64_t e1 = gld(v.l1, blk1);
+  const uint64_t r = i - (Value ? e1 : (blk1 << 16) - e1);
+  uint32_t below =
+      t != 0 && t <= span && (Value ? e0 : ((k_lo + t - first) << 9) - e0) < r ? 1u : 0u;
+  for (uint64_t u = t + G; u <= span; u += G) {
     const uint64_t k = k_lo + u;
     const uint64_t e = gld(v.l2, k);
     below += (Value ? e : ((k - first) << 9) - e) < r ? 1u : 0u;
   }
-  const uint64_t blk2 = k_lo + group_sum<G>(below);
-  const uint64_t e2 = gld(v.l2, blk2);
+  const uint32_t at = group_sum<G>(below);
+  const uint64_t blk2 = k_lo + at;
+  const uint32_t near = __shfl(static_cast<uint32_t>(e0), static_cast<int>(at % G), G);
+  const uint64_t e2 = at < G ? near : gld(v.l2, blk2);
   const uint64_t rr = r - (Value ? e2 : ((blk2 - first) << 9) - e2);
   return group_select_words<Value, G>(reinterpret_cast<const uint64_t*>(v.words + (blk2 << 4)),
                                       8, 0, rr, blk2 << 9, v.size);
