@@ -72,65 +72,95 @@ __device__ __forceinline__ uint64_t rs_num_l2(uint64_t m, uint64_t num_l1) {
   return m ? (num_l1 - 1) * detail::kL2PerL1 + last : 0;
 }
 
-// One thread per tree: from the digit-count rows at the text boundaries,
-// the tree's digit starts (pc, for the pass), its C array and node ranks
-// (wavelet_tree.cuh:773-774, 332-352: the zeros of level l before each node
-// start, in (level, symbol) order) and the sizes of its levels
-// (wavelet_tree.cuh:776-790) in its directory descriptors.
-__global__ void forest_meta_kernel(const uint64_t* __restrict__ rows, const MetaJob* __restrict__ jobs,
-                                   uint32_t N, const ShapeDev* __restrict__ shapes,
-                                   const uint8_t* __restrict__ sh_code,
-                                   const uint8_t* __restrict__ sh_len,
-                                   const uint16_t* __restrict__ sh_node,
-                                   const uint8_t* __restrict__ sh_node_level,
-                                   uint8_t* __restrict__ arena, uint64_t* __restrict__ pc,
-                                   RsArrayDesc* __restrict__ desc) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
+// exclusive scan over a workgroup of 256 threads; s_w holds 4 u64
+__device__ __forceinline__ uint64_t wg_excl_scan_u64(uint64_t v, uint64_t* s_w) {
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t incl = v;
+#pragma unroll
+  for (uint32_t off = 1; off < 64; off <<= 1) {
+    const uint64_t y = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += y;
+  }
+  __syncthreads();  // earlier readers of s_w are done
+  if (lane == 63) s_w[wave] = incl;
+  __syncthreads();
+  uint64_t before = 0;
+  for (uint32_t w = 0; w < wave; ++w) before += s_w[w];
+  return before + incl - v;
+}
+
+// One workgroup per tree, a thread per digit, symbol and node in turn: from
+// the digit-count rows at the text boundaries, the tree's digit starts (pc,
+// for the pass), its C array and node ranks (wavelet_tree.cuh:773-774,
+// 332-352: the zeros of level l before each node start, in (level, symbol)
+// order) and the sizes of its levels (wavelet_tree.cuh:776-790) in its
+// directory descriptors.  One thread per tree filled 16 workgroups for 2000
+// trees, each thread a chain of 700 loads: 193 us; now 17 us.
+static_assert(kRow == 256, "one thread per digit");
+__global__ __launch_bounds__(256) void forest_meta_kernel(
+    const uint64_t* __restrict__ rows, const MetaJob* __restrict__ jobs,
+    const ShapeDev* __restrict__ shapes, const uint8_t* __restrict__ sh_code,
+    const uint8_t* __restrict__ sh_len, const uint16_t* __restrict__ sh_node,
+    const uint8_t* __restrict__ sh_node_level, uint8_t* __restrict__ arena,
+    uint64_t* __restrict__ pc, RsArrayDesc* __restrict__ desc) {
+  __shared__ uint64_t s_w[4], s_cnt[kRow], s_C[kRow], s_m[8], s_first[8];
+  __shared__ uint32_t s_kw[4];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t i = blockIdx.x;
   const MetaJob J = jobs[i];
   const ShapeDev S = shapes[J.shape];
-  const uint64_t* r0 = rows + static_cast<uint64_t>(i) * kRow;
-  const uint64_t* r1 = r0 + kRow;
-  uint64_t* P = pc + static_cast<uint64_t>(i) * (kRow + 1);
-  uint64_t run = 0;
-  for (uint32_t d = 0; d < kRow; ++d) {
-    P[d] = run;
-    run += r1[d] - r0[d];
-  }
-  P[kRow] = run;
-  uint64_t* C = reinterpret_cast<uint64_t*>(arena + J.counts_at);
-  uint64_t m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  uint64_t acc = 0;
-  for (uint32_t c = 0; c < S.sigma; ++c) {
-    const uint8_t code = sh_code[S.code_off + c];
-    const uint64_t cnt = r1[code] - r0[code];
-    C[c] = acc;
-    acc += cnt;
-    const uint32_t len = sh_len[S.code_off + c];
-    for (uint32_t l = 0; l < 8; ++l)
-      if (l < len) m[l] += cnt;
-  }
-  uint64_t* R = reinterpret_cast<uint64_t*>(arena + J.ranks_at);
-  uint32_t k = 0, cur = 0xFFFFFFFFu;
-  uint64_t zb = 0;
-  for (uint32_t j = 0; j < S.nodes; ++j) {
-    const uint32_t lo = sh_node[2 * (S.node_off + j)], hi = sh_node[2 * (S.node_off + j) + 1];
-    const uint32_t l = sh_node_level[S.node_off + j];
-    if (l != cur) {
-      cur = l;
-      zb = 0;
-    }
-    const uint32_t mid = lo + static_cast<uint32_t>(detail::prev_pow2(hi - lo + 1));
-    if (l >= 1 && lo >= 1) R[k++] = zb;
-    const uint64_t cmid = mid < S.sigma ? C[mid] : J.n;
-    zb += cmid - C[lo];
-  }
+  // digits
+  const uint64_t cnt = rows[(i + 1) * kRow + tid] - rows[i * kRow + tid];
+  s_cnt[tid] = cnt;
+  if (tid < 8) s_m[tid] = 0;
+  const uint64_t start = wg_excl_scan_u64(cnt, s_w);
+  uint64_t* P = pc + i * (kRow + 1);
+  P[tid] = start;
+  if (tid == kRow - 1) P[kRow] = start + cnt;
+  // symbols: C, and the codes longer than l of every level l
+  const bool symbol = tid < S.sigma;
+  const uint64_t occ = symbol ? s_cnt[sh_code[S.code_off + tid]] : 0;
+  const uint32_t len = symbol ? sh_len[S.code_off + tid] : 0;
+  const uint64_t C = wg_excl_scan_u64(occ, s_w);
+  s_C[tid] = C;
+  if (symbol) reinterpret_cast<uint64_t*>(arena + J.counts_at)[tid] = C;
   for (uint32_t l = 0; l < S.L; ++l) {
-    RsArrayDesc& d = desc[J.desc0 + l];
-    d.m = m[l];
-    d.num_l1 = (m[l] + detail::kL1Bits - 1) / detail::kL1Bits;
-    d.num_l2 = rs_num_l2(m[l], d.num_l1);
-    d.cap = m[l] / detail::kSampleRate;
+    const uint64_t sum = detail::wave_sum_u64(l < len ? occ : 0);
+    if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long*>(&s_m[l]), sum);
+  }
+  __syncthreads();
+  // nodes, sorted by level: the zeros before each in its level
+  const bool node = tid < S.nodes;
+  uint32_t lo = 0, l = 0;
+  uint64_t zeros = 0;
+  bool ranked = false, heads = false;
+  if (node) {
+    const uint32_t j = S.node_off + tid;
+    lo = sh_node[2 * j];
+    const uint32_t hi = sh_node[2 * j + 1];
+    l = sh_node_level[j];
+    heads = tid == 0 || sh_node_level[j - 1] != l;
+    const uint32_t mid = lo + static_cast<uint32_t>(detail::prev_pow2(hi - lo + 1));
+    zeros = (mid < S.sigma ? s_C[mid] : J.n) - s_C[lo];
+    ranked = l >= 1 && lo >= 1;
+  }
+  const uint64_t ranked_lanes = detail::ballot64(ranked);
+  if (lane == 0) s_kw[wave] = static_cast<uint32_t>(__popcll(ranked_lanes));
+  const uint64_t before = wg_excl_scan_u64(zeros, s_w);
+  if (heads) s_first[l] = before;
+  __syncthreads();
+  if (ranked) {
+    uint32_t k = detail::mbcnt64(ranked_lanes);
+    for (uint32_t w = 0; w < wave; ++w) k += s_kw[w];
+    reinterpret_cast<uint64_t*>(arena + J.ranks_at)[k] = before - s_first[l];
+  }
+  if (tid < S.L) {
+    RsArrayDesc& d = desc[J.desc0 + tid];
+    const uint64_t m = s_m[tid];
+    d.m = m;
+    d.num_l1 = (m + detail::kL1Bits - 1) / detail::kL1Bits;
+    d.num_l2 = rs_num_l2(m, d.num_l1);
+    d.cap = m / detail::kSampleRate;
   }
 }
 
@@ -450,8 +480,8 @@ void enqueue_build(ecl_forest_t* f, ForestBuild& B, hipStream_t s) {
   launch_tile_scan(B.pp, s);
   launch_gather_rows(B.d_excl.as<uint64_t>(), B.d_tfirst.as<uint32_t>(), B.N + 1, kRow,
                      B.d_rows.as<uint64_t>(), s);
-  hipLaunchKernelGGL(forest_meta_kernel, dim3((B.N + 127) / 128), dim3(128), 0, s,
-                     B.d_rows.as<uint64_t>(), B.d_jobs.as<MetaJob>(), B.N,
+  hipLaunchKernelGGL(forest_meta_kernel, dim3(B.N), dim3(256), 0, s,
+                     B.d_rows.as<uint64_t>(), B.d_jobs.as<MetaJob>(),
                      B.d_shapes.as<ShapeDev>(), B.d_code.as<uint8_t>(), B.d_len.as<uint8_t>(),
                      B.d_node.as<uint16_t>(), B.d_node_level.as<uint8_t>(),
                      f->arena.as<uint8_t>(), B.d_pc.as<uint64_t>(), B.d_desc.as<RsArrayDesc>());
