@@ -117,19 +117,26 @@ __global__ __launch_bounds__(256) void histogram_kernel(HistParams p,
 //  2. rs_chunk_sum / rs_chunk_scan / rs_l1_write kernels: the exclusive scan
 //     of every array's block totals = its L1 entries, and its total (chunk
 //     sums, their scan per array, chunk scans from their bases).
-//  3. rs_samples_kernel: one wave per L1 block, one lane per select sample
+//  3. rs_samples_kernel: half a wave per L1 block, a lane per select sample
 //     that falls inside the block: binary search over the block's L2 entries,
 //     then one 64-byte L2 block is read and the bit is selected in-word.
 // Global L1 block g belongs to array block_array[g] (written by
 // rs_block_map_kernel), whose first block is arrays[...].first_tile.
 constexpr uint32_t kRsWaves = 8;  // L1 blocks per workgroup
 
-// one workgroup per array: its blocks' entries of block_array
+// one thread per L1 block: the last array whose first block is at or before
+// it (a workgroup per array had taken 29 us for one array of 2^18 blocks)
 __global__ __launch_bounds__(256) void rs_block_map_kernel(const RsArrayDesc* __restrict__ arrays,
+                                                           uint32_t narrays, uint64_t nblocks,
                                                            uint32_t* __restrict__ block_array) {
-  const RsArrayDesc& a = arrays[blockIdx.x];
-  const uint64_t first = a.first_tile, cnt = a.cap_l1 ? a.cap_l1 : a.num_l1;
-  for (uint64_t b = threadIdx.x; b < cnt; b += 256) block_array[first + b] = blockIdx.x;
+  const uint64_t b = blockIdx.x * 256ull + threadIdx.x;
+  if (b >= nblocks) return;
+  uint32_t lo = 0, hi = narrays;
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (arrays[mid].first_tile <= b) lo = mid; else hi = mid;
+  }
+  block_array[b] = lo;
 }
 
 __global__ __launch_bounds__(512) void rs_local_kernel(const RsArrayDesc* __restrict__ arrays,
@@ -299,14 +306,19 @@ __device__ __forceinline__ uint32_t select_in_block(const uint64_t* q, uint32_t 
   return at;
 }
 
+// Half a wave per L1 block: a block holds at most 18 samples (ones + zeros =
+// 65536 bits), and the kernel waits for its three loads in turn (entries,
+// then the L2 block), so it is bound by how many blocks are in flight: with a
+// wave per block 2^18 blocks took 329 us, now 250 us (their 8.4 * 10^6 random
+// 128-byte lines move at 4.3 TB/s).
 __global__ __launch_bounds__(512) void rs_samples_kernel(const RsArrayDesc* __restrict__ arrays,
                                                          const uint32_t* __restrict__ block_array,
                                                          uint64_t nblocks) {
-  __shared__ uint16_t s_l2[kRsWaves][detail::kL2PerL1];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint64_t gb = static_cast<uint64_t>(blockIdx.x) * kRsWaves + wave;
+  __shared__ __align__(16) uint16_t s_l2[2 * kRsWaves][detail::kL2PerL1];
+  const uint32_t tid = threadIdx.x, lane = tid & 31, half = tid >> 5;
+  const uint64_t gb = static_cast<uint64_t>(blockIdx.x) * 2 * kRsWaves + half;
   if (gb >= nblocks) return;
-  const RsArrayDesc p = arrays[block_array[gb]];
+  const RsArrayDesc& p = arrays[block_array[gb]];
   if (p.cap == 0) return;
   const uint64_t kb = gb - p.first_tile;
   if (kb >= p.num_l1) return;  // reserved past the array's size
@@ -314,8 +326,8 @@ __global__ __launch_bounds__(512) void rs_samples_kernel(const RsArrayDesc* __re
   const uint64_t bits = p.m - bits0 < detail::kL1Bits ? p.m - bits0 : detail::kL1Bits;
   const uint64_t nl2 = (bits + detail::kL2Bits - 1) / detail::kL2Bits;  // L2 blocks here
   // the block's L2 entries are loaded together with its L1 entries
-  for (uint32_t x = lane; x < detail::kL2PerL1; x += 64)
-    s_l2[wave][x] = x < nl2 ? p.l2[kb * detail::kL2PerL1 + x] : 0xFFFFu;
+  for (uint32_t x = lane; x < detail::kL2PerL1; x += 32)
+    s_l2[half][x] = x < nl2 ? p.l2[kb * detail::kL2PerL1 + x] : 0xFFFFu;
   const uint64_t o0 = p.l1[kb];
   const uint64_t o1 = kb + 1 < p.num_l1 ? p.l1[kb + 1] : *p.total_ones;
   const uint64_t z0 = bits0 - o0, z1 = bits0 + bits - o1;
@@ -325,7 +337,7 @@ __global__ __launch_bounds__(512) void rs_samples_kernel(const RsArrayDesc* __re
   const uint64_t n1 = last1 >= first1 ? last1 - first1 + 1 : 0;
   const uint64_t n0 = last0 >= first0 ? last0 - first0 + 1 : 0;
   if (n1 + n0 == 0) return;
-  // the wave's LDS writes complete before its reads (in-order LDS queue)
+  // the half's LDS writes complete before its reads (in-order LDS queue)
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   __builtin_amdgcn_wave_barrier();
   // lanes 0 .. n1-1: ones samples; n1 .. n1+n0-1: zeros samples (<= 32 in all)
@@ -337,10 +349,10 @@ __global__ __launch_bounds__(512) void rs_samples_kernel(const RsArrayDesc* __re
     uint32_t lo = 0, hi = static_cast<uint32_t>(nl2);
     while (hi - lo > 1) {
       const uint32_t mid = (lo + hi) >> 1;
-      const uint32_t before = one ? s_l2[wave][mid] : mid * 512u - s_l2[wave][mid];
+      const uint32_t before = one ? s_l2[half][mid] : mid * 512u - s_l2[half][mid];
       if (before < r) lo = mid; else hi = mid;
     }
-    const uint32_t before = one ? s_l2[wave][lo] : lo * 512u - s_l2[wave][lo];
+    const uint32_t before = one ? s_l2[half][lo] : lo * 512u - s_l2[half][lo];
     const uint64_t wb = (bits0 >> 6) + lo * 8ull;  // first word of the L2 block
     const uint64_t valid = p.m - (wb << 6);
     const uint32_t pos = one ? select_in_block<1>(p.words64 + wb, r - before, valid)
@@ -1861,20 +1873,20 @@ void launch_rs_build(const RsArrayDesc* arrays, uint64_t narrays, uint64_t nbloc
   uint32_t* block_array = scratch;
   uint32_t* block_ones = scratch + nblocks;
   ProfScope ps(K_RS_BUILD, s);
-  hipLaunchKernelGGL(rs_block_map_kernel, dim3(static_cast<uint32_t>(narrays)), dim3(256), 0, s,
-                     arrays, block_array);
+  const uint32_t na = static_cast<uint32_t>(narrays);
+  hipLaunchKernelGGL(rs_block_map_kernel, dim3(static_cast<uint32_t>((nblocks + 255) / 256)),
+                     dim3(256), 0, s, arrays, na, nblocks, block_array);
   ECL_HIP(hipGetLastError());
   hipLaunchKernelGGL(rs_local_kernel, dim3(static_cast<uint32_t>(groups)), dim3(512), 0, s,
                      arrays, block_array, nblocks, block_ones);
   ECL_HIP(hipGetLastError());
-  const uint32_t na = static_cast<uint32_t>(narrays);
   hipLaunchKernelGGL(rs_chunk_sum_kernel, dim3(static_cast<uint32_t>(nchunks)), dim3(256), 0, s,
                      arrays, na, block_ones);
   hipLaunchKernelGGL(rs_chunk_scan_kernel, dim3(na), dim3(64), 0, s, arrays);
   hipLaunchKernelGGL(rs_l1_write_kernel, dim3(static_cast<uint32_t>(nchunks)), dim3(256), 0, s,
                      arrays, na, block_ones);
   ECL_HIP(hipGetLastError());
-  hipLaunchKernelGGL(rs_samples_kernel, dim3(static_cast<uint32_t>(groups)), dim3(512), 0, s,
+  hipLaunchKernelGGL(rs_samples_kernel, dim3(static_cast<uint32_t>((groups + 1) / 2)), dim3(512), 0, s,
                      arrays, block_array, nblocks);
   ECL_HIP(hipGetLastError());
 }
