@@ -1000,12 +1000,15 @@ TreeMemory tree_memory(uint64_t n, uint64_t sigma, uint32_t L, int esize, bool h
   TreeMemory m;
   m.resident = per_level * L + scan + sigma * 64 + (n / 4096 + 4096) * 8 +
                10'000'000ull * 16;
-  // level order with padded nodes (the build's pad_cap) of codes of w bytes
-  auto pad = [&](uint64_t w) { return (n + (2 * sigma + 2) * (16 / w)) * w; };
+  // level order with padded nodes (the build's pad_cap).  Every buffer is as
+  // wide as the first pass's codes, although later passes write narrower
+  // ones: the reported sizes and what is admitted do not depend on that, and
+  // any pass's output fits any buffer.
+  const uint64_t pad = (n + (2 * sigma + 2) * (16 / b.cw)) * b.cw;
   m.text = host_text ? n * esize : 0;
-  m.x = identity ? 0 : (b.npasses > 2 ? pad(b.cw) : n * b.cw);
-  m.u = b.npasses > 1 ? pad(b.w[1]) : 0;
-  m.v = b.npasses > 2 && identity ? pad(b.w[2]) : 0;
+  m.x = identity ? 0 : (b.npasses > 2 ? pad : n * b.cw);
+  m.u = b.npasses > 1 ? pad : 0;
+  m.v = b.npasses > 2 && identity ? pad : 0;
   return m;
 }
 uint64_t tree_needed_bytes(uint64_t n, uint64_t sigma, uint32_t L, int esize, bool host_text) {
@@ -1293,11 +1296,11 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     // codes of w bytes a level order with padded nodes holds
     auto pad_cap = [&](uint64_t w) { return n + (2 * sigma + 2) * (16 / w); };
     if (!identity) buf_x.alloc((plan.npasses > 2 ? pad_cap(cw) : n) * cw, x_host);
-    if (plan.npasses > 1) buf_u.alloc(pad_cap(plan.w[1]) * plan.w[1], u_host);
-    if (plan.npasses > 2 && identity) buf_v.alloc(pad_cap(plan.w[2]) * plan.w[2], v_host);
+    if (plan.npasses > 1) buf_u.alloc(pad_cap(cw) * cw, u_host);
+    if (plan.npasses > 2 && identity) buf_v.alloc(pad_cap(cw) * cw, v_host);
     if ((!identity && (plan.npasses > 2 ? pad_cap(cw) : n) * cw != mem.x) ||
-        (plan.npasses > 1 ? pad_cap(plan.w[1]) * plan.w[1] : 0) != mem.u ||
-        (plan.npasses > 2 && identity ? pad_cap(plan.w[2]) * plan.w[2] : 0) != mem.v)
+        (plan.npasses > 1 ? pad_cap(cw) * cw : 0) != mem.u ||
+        (plan.npasses > 2 && identity ? pad_cap(cw) * cw : 0) != mem.v)
       throw Error(ECL_ERROR_INTERNAL, "code buffer sizes differ from the memory estimate");
     const uint32_t k0 = plan.k[0], nb0 = 1u << k0;
     const uint64_t tiles0 = (n + T0 - 1) / T0;
