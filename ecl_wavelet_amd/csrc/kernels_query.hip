@@ -999,9 +999,9 @@ void rank_hex(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t*
 // Measured on n = 5e8, sigma = 256 in us, one lane (a pair over lines), 8 and
 // 16 lanes per query.  Directory select: 8000 queries 82 / 40 / 40, 16000 75 /
 // 45 / 46, 30000 73 / 50 / 65 (one lane over hints 55, 51, 47); over select
-// lines: 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access over query lines: 15.1 / 11.5 / 10.9, 15.6 / 12 /
-// 12.8, 16.5 / 14.6 / 19.5; over the directory 8 lanes gain nothing past 2^13
-// (16000: 13.9 / 13.4 / 14.2).
+// lines 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access over query lines
+// 15.1 / 11.5 / 10.9, 15.6 / 12 / 12.8, 16.5 / 14.6 / 19.5; over the directory
+// 8 lanes gain nothing past 2^13 (16000: 13.9 / 13.4 / 14.2).
 constexpr uint64_t kGroup16Max = 1u << 13, kGroup8Max = 1u << 14;
 int group_lanes(uint64_t m, uint64_t max8) {
   return m <= kGroup16Max ? 16 : m <= max8 ? 8 : 0;
