@@ -465,6 +465,7 @@ class WaveletTree:
 
     # ---- host batch queries
     def access(self, indices, flags=0):
+        """The symbols at the indices; 0 for an index past the text."""
         idx = np.ascontiguousarray(indices, dtype=np.uint64)
         out = np.empty(len(idx), dtype=self.dtype)
         call("ecl_wavelet_tree_access", self._h, _p(idx), len(idx), _p(out), flags)

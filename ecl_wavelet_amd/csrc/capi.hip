@@ -2858,7 +2858,10 @@ ecl_status ecl_wavelet_tree_access(ecl_wavelet_tree wt, const uint64_t* idx, siz
     require(wt && (m == 0 || (idx && out)), "NULL argument");
     if (m == 0) return;
     set_device(wt->device);
-    const TreeQueryParams p = query_params(wt, flags);
+    TreeQueryParams p = query_params(wt, flags);
+    // the slots hold whatever batch of whichever tree came before, and are
+    // copied out whole
+    p.zero_skipped = 1;
     pipelined(wt, idx, 8, out, wt->esize, m, "access",
               [&](void* din, size_t len, void* dout, hipStream_t st) {
                 launch_tree_access(p, static_cast<uint64_t*>(din), len, dout, st);

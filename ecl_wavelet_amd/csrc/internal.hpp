@@ -339,6 +339,8 @@ struct TreeQueryParams {
   int has_sel_lines;         // 1: the tree's levels carry select lines
   uint32_t lanes;            // lanes per access/rank query: 0 (the library-wide
                              // setting), 1 or 2 (the tree's own, from its tuner)
+  int zero_skipped;          // access: 1 writes 0 for an index past the text, 0 leaves
+                             // its output as it is
 };
 void launch_tree_access(const TreeQueryParams& p, const uint64_t* idx,
                         uint64_t m, void* out, hipStream_t s);

@@ -124,7 +124,10 @@ __global__ __launch_bounds__(256) void tree_access_kernel(
   for (uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / G;
        q < m; q += stride) {
     const uint64_t i = idx[q];
-    if (i >= p.view.n) continue;  // accessKernel skips such indices
+    if (i >= p.view.n) {  // accessKernel skips such indices
+      if (p.zero_skipped && (G == 1 || (threadIdx.x & 1) == 0)) out[q] = 0;
+      continue;
+    }
     const uint64_t r =
         detail::tree_access<G == 2>(p.view, mt.lv, mt.counts, mt.ranks, mt.nal, i);
     if (G == 1 || (threadIdx.x & 1) == 0) out[q] = amap ? amap[r] : static_cast<T>(r);
@@ -171,7 +174,11 @@ __global__ __launch_bounds__(256) void tree_access_group_kernel(
   const uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / G;
   const uint64_t i = q < m ? idx[q] : ~0ull;
   const Meta mt = stage_meta(p.view, s_meta);
-  if (i >= p.view.n) return;
+  if (q >= m) return;
+  if (i >= p.view.n) {
+    if (p.zero_skipped && threadIdx.x % G == 0) out[q] = 0;
+    return;
+  }
   const T* amap = static_cast<const T*>(p.alphabet_out);
   const uint64_t r = detail::tree_access<false, G>(p.view, mt.lv, mt.counts, mt.ranks, mt.nal, i);
   if (threadIdx.x % G == 0) out[q] = amap ? amap[r] : static_cast<T>(r);
@@ -239,7 +246,10 @@ __global__ __launch_bounds__(256) void tree_access_quad_kernel(
   for (uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / 2;
        q < m; q += stride) {
     const uint64_t i = idx[q];
-    if (i >= p.view.n) continue;  // accessKernel skips such indices (both lanes)
+    if (i >= p.view.n) {  // accessKernel skips such indices (both lanes)
+      if (p.zero_skipped && (threadIdx.x & 1) == 0) out[q] = 0;
+      continue;
+    }
     const uint64_t N = quad_access(p, base, i);
     if ((threadIdx.x & 1) == 0) out[q] = amap ? amap[N] : static_cast<T>(N);
   }
@@ -292,7 +302,10 @@ __global__ __launch_bounds__(256) void tree_access_hex_kernel(
   for (uint64_t q = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / 2;
        q < m; q += stride) {
     const uint64_t i = idx[q];
-    if (i >= p.view.n) continue;  // accessKernel skips such indices (both lanes)
+    if (i >= p.view.n) {  // accessKernel skips such indices (both lanes)
+      if (p.zero_skipped && (threadIdx.x & 1) == 0) out[q] = 0;
+      continue;
+    }
     const uint64_t N = hex_access(p, tab, i);
     if ((threadIdx.x & 1) == 0) out[q] = amap ? amap[N] : static_cast<T>(N);
   }

@@ -418,7 +418,9 @@ size_t ecl_wavelet_tree_needed_gpu_memory(size_t data_size, size_t alphabet_size
 
 /* Host batch queries (access :956-1231, rank :1247-1551, select :1567-1797).
  * Inputs and outputs are host arrays owned by the caller.  access writes
- * sizeof(T)-byte symbols (original alphabet unless ECL_RESULTS_MINIMAL);
+ * sizeof(T)-byte symbols (original alphabet unless ECL_RESULTS_MINIMAL), and
+ * 0 for an index past the text (accessKernel skips it: the device form below
+ * leaves that output as it was);
  * rank/select read ecl_rank_select_query[] (original-alphabet symbols unless
  * ECL_SYMBOLS_MINIMAL) and write u64 results. */
 ecl_status ecl_wavelet_tree_access(ecl_wavelet_tree wt, const uint64_t* indices, size_t m,

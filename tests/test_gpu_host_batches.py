@@ -63,3 +63,31 @@ def test_threads_and_released_buffers(gpu, tree):
     assert not failed, failed[0]
     release_cached_memory()
     _check(tree, 1000, 5)
+
+
+@pytest.mark.parametrize("stage", ["directory", "query lines", "quad", "hex"])
+@pytest.mark.parametrize("dt", [np.uint8, np.uint16, np.uint64])
+def test_access_past_the_text_gives_zero(gpu, dt, stage):
+    """An index past the text has no symbol: its answer is 0, whatever batch
+    of another tree the shared staging slots held before.  Batch sizes of
+    every access kernel (16, 8, 2 and 1 lanes per query) and of a pipelined
+    batch."""
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(5)
+    n, sigma = 70_003, 16
+    alphabet = np.arange(3, 3 + sigma).astype(dt)  # no symbol is 0
+    text = alphabet[rng.integers(0, sigma, n)]
+    wt = WaveletTree(text, alphabet)
+    {"directory": lambda: None, "query lines": wt.buildQueryLines, "quad": wt.buildQuadLines,
+     "hex": wt.buildHexLines}[stage]()
+    other = WaveletTree(np.full(5000, 1, np.uint8), np.arange(2, dtype=np.uint8))
+    for m in (1, 500, 8193, 40_000, 4 * CHUNK + 3):
+        # every staged output byte of the other tree's batch is not 0
+        q = other.make_queries(np.full(m, 4369), np.full(m, 1))
+        assert np.all(other.rank(q) == 4369)
+        idx = rng.integers(0, n, m).astype(np.uint64)
+        past = rng.random(m) < 0.3
+        past[m // 2] = True
+        idx[past] = rng.choice(np.array([n, n + 1, 1 << 40, 2**64 - 1], np.uint64), past.sum())
+        want = np.where(past, dt(0), text[np.where(past, 0, idx).astype(np.int64)])
+        assert np.array_equal(wt.access(idx), want), m
