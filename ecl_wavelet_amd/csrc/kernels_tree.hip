@@ -186,7 +186,8 @@ __global__ __launch_bounds__(kPassThreads) void tile_hist_kernel(PassParams p) {
   using Code = typename CodeOf<CW>::type;
   const uint32_t T = p.tile_codes;                   // codes per tile
   constexpr uint32_t EI = 16 / sizeof(TIn);          // input symbols per chunk
-  __shared__ uint32_t s_bins[kHistSlots];
+  __shared__ __align__(16) uint32_t s_bins[kHistSlots];  // cleared by 16-byte stores
+  static_assert(__alignof__(s_bins) >= 16, "the bins are cleared as uint4");
   __shared__ uint32_t s_tot[kMaxBins];
   __shared__ uint8_t s_map[Remap && sizeof(TIn) == 1 ? 256 : 1];  // symbol -> code
   const uint32_t tid = threadIdx.x;
@@ -777,7 +778,9 @@ void pass_kernel(PassParams p) {
   __shared__ uint64_t s_gR[kLevelGroups];          // group destination bit
   __shared__ uint32_t s_gSL[kLevelGroups];         // group tile start | length << 16
   __shared__ uint32_t s_gw[kLevelGw];              // full destination words before each group
-  __shared__ uint16_t s_base[kLevelChildren];      // partition base per child
+  // partition base per child; a group's two children are read as one word
+  __shared__ __align__(4) uint16_t s_base[kLevelChildren];
+  static_assert(__alignof__(s_base) >= 4, "pairs of bases are words");
   __shared__ uint64_t s_cD[kLevelGroups];          // carried word (index into p.words)
   __shared__ uint32_t s_cV[kLevelGroups];          // its bits so far
   __shared__ uint8_t s_cLo[kLevelGroups];          // first of them; kNoCarry: none
