@@ -1287,6 +1287,10 @@ void launch_pass(const PassParams& params, hipStream_t s) {
   const dim3 grid(static_cast<uint32_t>((p.num_tiles + span - 1) / span)), block(kPassThreads);
   if (p.tile_codes != pass_tile_codes(p.cw, p.tile_rows))
     throw Error(ECL_ERROR_INTERNAL, "tile size does not match the tile rows");
+  // the kernel narrows its codes or keeps their width (write_codes)
+  if (p.dst != nullptr && ((p.dst_cw != 1 && p.dst_cw != 2 && p.dst_cw != 4 && p.dst_cw != 8) ||
+                           p.dst_cw > p.cw))
+    throw Error(ECL_ERROR_INTERNAL, "a pass cannot write codes of this width");
 #define ECL_PASS_ROWS(CWV)                                                                  \
   do {                                                                                      \
     if (p.tile_rows == 4) hipLaunchKernelGGL((pass_kernel<CWV, 4>), grid, block, 0, s, p);  \
