@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "host.hpp"
+#include "host_pipes.hpp"
 
 using ecl::detail::LevelView;
 using ecl::detail::TreeView;
@@ -302,7 +303,7 @@ void upload_staged(void* d_dst, const void* src, size_t bytes, hipStream_t s) {
   Staging& st = *g_staging;
   std::lock_guard<std::mutex> lk(st.mu);
   for (int b = 0; b < 2; ++b) {
-    if (!st.pin[b]) ECL_HIP(hipHostMalloc(&st.pin[b], kStageBytes, hipHostMallocDefault));
+    if (!st.pin[b]) st.pin[b] = alloc_pinned(kStageBytes);
     if (!st.done[b]) ECL_HIP(hipEventCreateWithFlags(&st.done[b], hipEventDisableTiming));
   }
   auto* d = static_cast<uint8_t*>(d_dst);
@@ -481,75 +482,41 @@ static hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 // ===========================================================================
 // host-issued batches
 // ===========================================================================
-// A pipe is what one host-issued batch call works with: kPipeSlots
-// default-priority streams, each with pinned input and output buffers grown
-// on demand.  Calls take an idle pipe of their device (or make one) and put
-// it back, so a tree's first call does not pay for streams and pinned memory
-// (about 0.45 ms to make and unmake for a tree that is asked three times),
-// and calls from several threads, on one tree or many, have a pipe each.  At
-// most kIdlePipes wait per device; ecl_release_cached_memory gives them back.
+// A call takes an idle pipe of its device (or makes one) and puts it back, so
+// a tree's first call does not pay for streams and pinned memory (about 0.45
+// ms to make and unmake for a tree that is asked three times), and calls from
+// several threads, on one tree or many, have a pipe each.  The streams have
+// the default priority.  ecl_release_cached_memory gives the idle pipes back,
+// and so does any pinned allocation of the library that would fail.
 namespace ecl {
 namespace lib {
 namespace {
-constexpr int kPipeSlots = 3;
-constexpr size_t kIdlePipes = 4;
-constexpr size_t kPipeMinBytes = size_t(1) << 20;  // smallest buffer of a slot
-constexpr int kPipeDevices = 64;
-
-struct HostPipe {
-  int device = 0;
-  hipStream_t stream[kPipeSlots] = {};
-  void* pin_in[kPipeSlots] = {};
-  void* pin_out[kPipeSlots] = {};
-  size_t cap_in[kPipeSlots] = {}, cap_out[kPipeSlots] = {};
-  ~HostPipe() {
-    for (int i = 0; i < kPipeSlots; ++i) {
-      if (stream[i]) (void)hipStreamDestroy(stream[i]);
-      if (pin_in[i]) (void)hipHostFree(pin_in[i]);
-      if (pin_out[i]) (void)hipHostFree(pin_out[i]);
-    }
+struct HipRuntime {
+  using Stream = hipStream_t;
+  using Error = hipError_t;
+  using DeviceScope = ecl::lib::DeviceScope;
+  static constexpr hipError_t kOk = hipSuccess;
+  static void check(hipError_t e, const char* what) { hip_check(e, what); }
+  static hipError_t stream_create(hipStream_t* s) { return hipStreamCreate(s); }
+  static void stream_destroy(hipStream_t s) { (void)hipStreamDestroy(s); }
+  static hipError_t pinned_alloc(void** p, size_t bytes) {
+    const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
   }
-  static void grow(void*& pin, size_t& cap, size_t bytes) {
-    if (bytes <= cap) return;
-    if (pin) ECL_HIP(hipHostFree(pin));
-    pin = nullptr;
-    cap = 0;
-    bytes = std::max(bytes, kPipeMinBytes);
-    ECL_HIP(hipHostMalloc(&pin, bytes, hipHostMallocDefault));
-    cap = bytes;
-  }
-  void reserve(int slots, size_t in_bytes, size_t out_bytes) {
-    for (int i = 0; i < slots; ++i) {
-      if (!stream[i]) ECL_HIP(hipStreamCreate(&stream[i]));
-      grow(pin_in[i], cap_in[i], in_bytes);
-      grow(pin_out[i], cap_out[i], out_bytes);
-    }
-  }
-};
-
-struct PipePool {
-  std::mutex mu;
-  std::vector<std::unique_ptr<HostPipe>> idle;
+  static void pinned_free(void* p) { (void)hipHostFree(p); }
 };
 // never destroyed: see g_pool
-PipePool* const g_pipes = new PipePool[kPipeDevices];
+PipePool<HipRuntime>& pipes() {
+  static auto* const pool = new PipePool<HipRuntime>();
+  return *pool;
+}
 
 // a pipe of the device for the length of one call; one whose call failed is
 // not handed on
 class PipeLease {
  public:
-  explicit PipeLease(int device) {
-    if (device >= 0 && device < kPipeDevices) {
-      PipePool& P = g_pipes[device];
-      std::lock_guard<std::mutex> lk(P.mu);
-      if (!P.idle.empty()) {
-        pipe_ = std::move(P.idle.back());
-        P.idle.pop_back();
-      }
-    }
-    if (!pipe_) pipe_.reset(new HostPipe());
-    pipe_->device = device;
-  }
+  explicit PipeLease(int device) : pipe_(pipes().take(device)) {}
   ~PipeLease() {
     if (!done_) {  // its kernels may still run
       for (hipStream_t st : pipe_->stream)
@@ -557,38 +524,25 @@ class PipeLease {
       (void)hipGetLastError();
       return;
     }
-    const int device = pipe_->device;
-    if (device < 0 || device >= kPipeDevices) return;
-    PipePool& P = g_pipes[device];
-    std::unique_lock<std::mutex> lk(P.mu);
-    if (P.idle.size() < kIdlePipes) {
-      P.idle.push_back(std::move(pipe_));
-    } else {
-      lk.unlock();
-      pipe_.reset();
-    }
+    pipes().give(std::move(pipe_));
   }
   PipeLease(const PipeLease&) = delete;
   PipeLease& operator=(const PipeLease&) = delete;
-  HostPipe* operator->() const { return pipe_.get(); }
+  HostPipe<HipRuntime>* operator->() const { return pipe_.get(); }
+  void reserve(int slots, size_t in_bytes, size_t out_bytes) {
+    pipe_->reserve(pipes(), slots, in_bytes, out_bytes);
+  }
   void done() { done_ = true; }  // every stream of the pipe is idle
 
  private:
-  std::unique_ptr<HostPipe> pipe_;
+  std::unique_ptr<HostPipe<HipRuntime>> pipe_;
   bool done_ = false;
 };
 }  // namespace
 
-void release_host_pipes(int device) {
-  if (device < 0 || device >= kPipeDevices) return;
-  std::vector<std::unique_ptr<HostPipe>> gone;
-  {
-    std::lock_guard<std::mutex> lk(g_pipes[device].mu);
-    gone.swap(g_pipes[device].idle);
-  }
-  DeviceScope ds(device);
-  gone.clear();
-}
+void* alloc_pinned(size_t bytes) { return pipes().alloc_pinned(bytes); }
+void release_host_pipes(int device) { pipes().release(device); }
+void release_all_host_pipes() { pipes().release_all(); }
 }  // namespace lib
 }  // namespace ecl
 
@@ -1030,7 +984,7 @@ struct StagingBuf {
     reset();
     if (bytes == 0) return;
     if (on_host) {
-      ECL_HIP(hipHostMalloc(&host, bytes, hipHostMallocDefault));
+      host = alloc_pinned(bytes);
       ptr = host;
     } else {
       dev = DevBuf(bytes);
@@ -1237,8 +1191,11 @@ static ecl_wavelet_tree_t* build_tree(int esize, const void* text, bool text_on_
     const bool x_host = on_host(mem.x);
     const bool u_host = on_host(mem.u);
     const bool v_host = on_host(mem.v);
-    if (host_bytes > available_host_memory())
-      throw Error(ECL_ERROR_OUT_OF_MEMORY_TREE, kOomTree);
+    if (host_bytes > available_host_memory()) {
+      release_all_host_pipes();  // idle staging is not a reason to refuse
+      if (host_bytes > available_host_memory())
+        throw Error(ECL_ERROR_OUT_OF_MEMORY_TREE, kOomTree);
+    }
     wt->build_host_bytes = host_bytes;
 
     // ---- the text on the device (or in pinned host memory)
@@ -2776,8 +2733,8 @@ static void pipelined(ecl_wavelet_tree wt, const void* in, size_t in_elem, void*
   const uint64_t need = 2 * std::min<uint64_t>(m, kHostChunk / 4) * (in_elem + out_elem);
   if (nchunks > 1) check_query_memory(need, kind);
   PipeLease P(wt->device);
-  P->reserve(static_cast<int>(std::min<size_t>(nchunks, kPipeSlots)), chunk * in_elem,
-             chunk * out_elem);
+  P.reserve(static_cast<int>(std::min<size_t>(nchunks, kPipeSlots)), chunk * in_elem,
+            chunk * out_elem);
   const auto* src = static_cast<const uint8_t*>(in);
   auto* dst = static_cast<uint8_t*>(out);
   auto put = [&](size_t c) {

@@ -67,8 +67,12 @@ constexpr size_t kPoolMinBytes = size_t(1) << 20;
 size_t pooled_bytes(int device);
 // frees every cached block of the device
 void release_block_pool(int device);
-// frees the idle pinned buffers of the host query calls (capi.hip)
+// frees the idle pinned buffers of the host query calls (capi.hip), of one
+// device or of all
 void release_host_pipes(int device);
+void release_all_host_pipes();
+// pinned host memory; the idle pinned buffers are freed before it fails
+void* alloc_pinned(size_t bytes);
 
 // ---- kernel profiling (events around selected launches) -------------------
 enum KernelId : int {

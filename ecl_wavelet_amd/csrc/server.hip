@@ -320,15 +320,10 @@ ecl_status ecl_server_create(int device, const ecl_server_config* config, ecl_se
       auto sl = std::make_unique<Slot>();
       ECL_HIP(hipStreamCreateWithFlags(&sl->stream, hipStreamNonBlocking));
       ECL_HIP(hipEventCreateWithFlags(&sl->done, hipEventDisableTiming));
-      void* p = nullptr;
-      ECL_HIP(hipHostMalloc(&p, B * sizeof(ecl_query), hipHostMallocDefault));
-      sl->pin_q = static_cast<ecl_query*>(p);
-      ECL_HIP(hipHostMalloc(&p, kMaxSegments * 8ull, hipHostMallocDefault));
-      sl->pin_seg = static_cast<uint64_t*>(p);
-      ECL_HIP(hipHostMalloc(&p, kMaxSegments * 4ull, hipHostMallocDefault));
-      sl->pin_tree = static_cast<uint32_t*>(p);
-      ECL_HIP(hipHostMalloc(&p, B * 8, hipHostMallocDefault));
-      sl->pin_out = static_cast<uint64_t*>(p);
+      sl->pin_q = static_cast<ecl_query*>(alloc_pinned(B * sizeof(ecl_query)));
+      sl->pin_seg = static_cast<uint64_t*>(alloc_pinned(kMaxSegments * 8ull));
+      sl->pin_tree = static_cast<uint32_t*>(alloc_pinned(kMaxSegments * 4ull));
+      sl->pin_out = static_cast<uint64_t*>(alloc_pinned(B * 8));
       sl->d_q = DevBuf(B * sizeof(ecl_query));
       sl->d_seg = DevBuf(kMaxSegments * 8ull);
       sl->d_tree = DevBuf(kMaxSegments * 4ull);

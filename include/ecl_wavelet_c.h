@@ -117,7 +117,8 @@ ecl_status ecl_device_mem_info(int device, size_t* free_bytes, size_t* total_byt
  * the device's memory; freed when an allocation would fail), keeps the
  * construction scratch (tile histograms and their scan, about 0.1 bytes per
  * symbol) for the next build, and keeps up to four idle sets of the host
- * query calls' staging buffers (each at most 36 MB of pinned host memory).
+ * query calls' staging buffers (each at most 36 MiB of pinned host memory;
+ * freed when a pinned allocation would fail).
  * This frees all three.
  * No counterpart in the reference, which allocates and frees per call; for
  * callers that need the memory back outside the library. */

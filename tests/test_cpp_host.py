@@ -10,7 +10,7 @@ from ecl_wavelet_amd import build
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-@pytest.mark.parametrize("name", ["test_pass_params"])
+@pytest.mark.parametrize("name", ["test_host_pipes", "test_pass_params"])
 def test_cpp_host(tmp_path, name):
     exe = str(tmp_path / name)
     cmd = [build.hipcc(), *build.common_flags(), "-x", "hip",
