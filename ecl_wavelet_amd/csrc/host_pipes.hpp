@@ -14,9 +14,12 @@ namespace lib {
 constexpr int kPipeSlots = 3;
 constexpr int kPipeDevices = 64;
 constexpr size_t kPipeMinBytes = size_t(1) << 20;  // smallest buffer of a slot
-// Idle pipes kept per device.  A pipe has at most 36 MiB pinned (3 slots of
-// 2^19 queries of 16 bytes and results of 8).
-constexpr size_t kIdlePipes = 4;
+// Idle pipes kept per device: as many as may call at once without a pipe
+// being made and unmade per call.  With four, 16 threads took twice as long
+// as with a pipe per tree (rank batches of 10^5: 44 -> 78 us each).  A pipe
+// has at most 36 MB pinned (3 slots of 2^19 queries of 16 bytes and results
+// of 8), so 32 of them 1.2 GB; a pipe per tree had pinned 192 MB each.
+constexpr size_t kIdlePipes = 32;
 
 // Rt: Stream; Error, kOk and check(e, what), which throws for others;
 // stream_create(Stream*), stream_destroy(Stream), pinned_alloc(void**,

@@ -116,7 +116,7 @@ ecl_status ecl_device_mem_info(int device, size_t* free_bytes, size_t* total_byt
  * hands them out again for requests of the same size class (up to 40% of
  * the device's memory; freed when an allocation would fail), keeps the
  * construction scratch (tile histograms and their scan, about 0.1 bytes per
- * symbol) for the next build, and keeps up to four idle sets of the host
+ * symbol) for the next build, and keeps up to 32 idle sets of the host
  * query calls' staging buffers (each at most 36 MiB of pinned host memory;
  * freed when a pinned allocation would fail).
  * This frees all three.

@@ -1,6 +1,6 @@
 // The pool of host pipes over a counting runtime with a limited amount of
-// pinned memory: what idle pipes are kept and what gives them back.  Host
-// code only.
+// pinned memory: what idle pipes are kept, what gives them back, and that
+// many callers at once do not make and unmake pipes.  Host code only.
 #include <atomic>
 #include <condition_variable>
 #include <cstdio>
@@ -138,6 +138,35 @@ int main() {
     Fake::limit = ~size_t(0);
   }
   EXPECT(Fake::pinned == 0 && Fake::streams == 0);
+  {  // 16 callers at once, again and again: no pipe is made after the first round
+    Pool pool;
+    constexpr int kThreads = 16, kRounds = 50;
+    std::mutex mu;
+    std::condition_variable cv;
+    int arrived = 0;
+    int made_first = 0;
+    auto barrier = [&](int round) {
+      std::unique_lock<std::mutex> lk(mu);
+      ++arrived;
+      if (arrived == kThreads * round) cv.notify_all();
+      cv.wait(lk, [&] { return arrived >= kThreads * round; });
+    };
+    Fake::streams_made = 0;
+    std::vector<std::thread> th;
+    for (int t = 0; t < kThreads; ++t)
+      th.emplace_back([&, t] {
+        for (int r = 0; r < kRounds; ++r) {
+          auto p = pool.take(0);
+          p->reserve(pool, 3, MiB, MiB);
+          barrier(2 * r + 1);  // all of them hold one
+          if (t == 0 && r == 0) made_first = Fake::streams_made;
+          pool.give(std::move(p));
+          barrier(2 * r + 2);
+        }
+      });
+    for (auto& t : th) t.join();
+    EXPECT(made_first == 3 * kThreads && Fake::streams_made == made_first);
+  }
   EXPECT(Fake::pinned == 0 && Fake::streams == 0 && Fake::bad_frees == 0);
   std::printf(g_bad ? "FAILED\n" : "ALL OK\n");
   return g_bad != 0;
