@@ -91,3 +91,36 @@ def test_access_past_the_text_gives_zero(gpu, dt, stage):
         idx[past] = rng.choice(np.array([n, n + 1, 1 << 40, 2**64 - 1], np.uint64), past.sum())
         want = np.where(past, dt(0), text[np.where(past, 0, idx).astype(np.int64)])
         assert np.array_equal(wt.access(idx), want), m
+
+
+@pytest.mark.parametrize("m", [1, 1000, CHUNK, CHUNK + 1])
+def test_refused_batch_launches_nothing(gpu, tree, m):
+    """A host batch is refused for device memory before its kernels run,
+    whatever its size, and its output is untouched."""
+    import ctypes as C
+
+    from ecl_wavelet_amd import Profiler, _lib, set_device_memory_cap
+    wt, text, _ = tree
+    idx = np.zeros(m, np.uint64)
+    q = wt.make_queries(np.ones(m), np.full(m, 3))
+    calls = {"access": (idx, np.full(m, 0xA5, np.uint8), 2 * m * 9),
+             "rank": (q, np.full(m, 0xA5, np.uint64), 2 * m * 24),
+             "select": (q, np.full(m, 0xA5, np.uint64), 2 * m * 24)}
+    try:
+        Profiler.enable()
+        for kind, (src, out, need) in calls.items():
+            args = (f"ecl_wavelet_tree_{kind}", wt._h, src.ctypes.data_as(C.c_void_p), m,
+                    out.ctypes.data_as(C.c_void_p), 0)
+            set_device_memory_cap(0, need - 1)
+            Profiler.reset()
+            with pytest.raises(_lib.EclError) as e:
+                _lib.call(*args)
+            assert e.value.status == _lib.ECL_ERROR_OUT_OF_MEMORY_QUERIES
+            assert Profiler.get("wt_" + kind)[0] == 0
+            assert np.all(out == 0xA5)
+            set_device_memory_cap(0, need)  # just enough
+            _lib.call(*args)
+            assert Profiler.get("wt_" + kind)[0] >= 1
+    finally:
+        Profiler.enable(False)
+        set_device_memory_cap(0, 0)
