@@ -164,9 +164,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void t
 // chain of line latencies, and in one lane the instructions between them (at
 // 1000 queries per wave slot the directory select spent 7.5 us a level).
 // With the work of a level spread over lanes, n = 5e8, sigma = 256, 1000
-// queries, directory: access 10.3 -> 9.1, rank 11.3 -> 10.3, select 60 -> 27
-// us; query and select lines: 13.5 -> 8.8, 15.3 -> 9.6, 27.5 -> 17.4 us; 2^16
-// symbols, n = 5e7: select 150 -> 51 and 108 -> 37 us.
+// queries: directory select 60 -> 27 us; query and select lines: access 13.5
+// -> 8.8, rank 15.3 -> 9.6, select 27.5 -> 17.4 us; 2^16 symbols, n = 5e7:
+// select 150 -> 51 and 108 -> 37 us.  Access and rank over the directory gain
+// at few sizes (group_lanes below).
 template <typename T, int G>
 __global__ __launch_bounds__(256) void tree_access_group_kernel(
     TreeQueryParams p, const uint64_t* __restrict__ idx, uint64_t m, T* __restrict__ out) {
@@ -1007,21 +1008,41 @@ void rank_hex(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t*
   }
 }
 
-// Lanes per query of a short batch over the binary levels: 16 up to 2^13
-// queries, 8 up to `max8` (0: none), then 0 (the kernels for throughput).
-// Measured on n = 5e8, sigma = 256 in us, one lane (a pair over lines), 8 and
-// 16 lanes per query.  Directory select: 8000 queries 82 / 40 / 40, 16000 75 /
-// 45 / 46, 30000 73 / 50 / 65 (one lane over hints 55, 51, 47); over select
-// lines 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access over query lines
-// 15.1 / 11.5 / 10.9, 15.6 / 12 / 12.8, 16.5 / 14.6 / 19.5; over the directory
-// 8 lanes gain nothing past 2^13 (16000: 13.9 / 13.4 / 14.2).
+// Lanes per query of a short batch over the binary levels (0: the kernels for
+// throughput).
+//
+// Selects, and access and rank over query lines: 16 up to 2^13 queries, 8 up
+// to `max8`.  Measured on n = 5e8, sigma = 256 in us, one lane (a pair over
+// lines), 8 and 16 lanes per query.  Directory select: 8000 queries 82 / 40 /
+// 40, 16000 75 / 45 / 46, 30000 73 / 50 / 65 (one lane over hints 55, 51,
+// 47); over select lines 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access
+// over query lines 15.1 / 11.5 / 10.9, 15.6 / 12 / 12.8, 16.5 / 14.6 / 19.5.
+// With few levels the launch is most of the time and the lanes make no
+// difference (n = 5e7 over lines, 8192 queries, a pair and 16 lanes: sigma = 2
+// 5.5 / 5.5, sigma = 4 5.9 / 5.7, sigma = 20 10.2 / 7.6 us).
 constexpr uint64_t kGroup16Max = 1u << 13, kGroup8Max = 1u << 14;
 int group_lanes(uint64_t m, uint64_t max8) {
   return m <= kGroup16Max ? 16 : m <= max8 ? 8 : 0;
 }
-// access and rank: not when the caller has set the lanes per query
-int group_lanes(const TreeQueryParams& p, uint64_t m, uint64_t max8) {
-  return p.lanes != 0 || g_query_lanes.load() != 0 ? 0 : group_lanes(m, max8);
+// Access and rank; not when the tree's lanes per query are set (by its caller
+// or by its tuner) or the library's.  Over the directory a level is a chain
+// of few instructions in one lane too, so 16 lanes gain only where many lines
+// come from HBM at once: from 128 to 512 queries over levels past the L2
+// caches, and over levels past the 256 MB cache up to 2^13 queries (rank: only
+// above 2^12).  16 lanes over one, time per batch (20 batches in turn): n =
+// 1e6, sigma = 256 1.05 to 1.14 at every size; n = 2e8: 1 query 1.05 (access)
+// and 1.13 (rank), 32 1.07 and 1.11, 128 0.88 and 0.91, 300 0.78 and 0.80,
+// 1000 to 8192 0.97 to 1.01; n = 4e9: 8192 0.80; sigma = 65536, n = 5e8: 4096
+// 0.80 and 1.03, 8192 0.81 and 0.98.
+constexpr uint64_t kDirGroupMin = 128, kDirGroupMax = 512, kDirRankMin = (1u << 12) + 1;
+constexpr uint64_t kDirGroupBytes = 1ull << 24, kDirGroupBytesLarge = 1ull << 29;
+int group_lanes(const TreeQueryParams& p, uint64_t m, bool rank) {
+  if (p.lanes != 0 || g_query_lanes.load() != 0) return 0;
+  if (p.has_lines) return group_lanes(m, kGroup8Max);
+  const uint64_t bytes = p.view.n / 8 * p.view.num_levels;
+  if (m < kDirGroupMin || m > kGroup16Max || bytes < kDirGroupBytes) return 0;
+  if (m <= kDirGroupMax) return 16;
+  return bytes >= kDirGroupBytesLarge && (!rank || m >= kDirRankMin) ? 16 : 0;
 }
 
 template <int G>
@@ -1071,7 +1092,7 @@ void launch_tree_access(const TreeQueryParams& p, const uint64_t* idx,
   } else if (p.quad.levels) {
     if (p.quad.nbase <= kQuadLdsBase) access_quad<true>(p, idx, m, out, s);
     else access_quad<false>(p, idx, m, out, s);
-  } else if (const int g = group_lanes(p, m, p.has_lines ? kGroup8Max : 0)) {
+  } else if (const int g = group_lanes(p, m, false)) {
     if (g == 16) access_group<16>(p, idx, m, out, s);
     else access_group<8>(p, idx, m, out, s);
   } else if (pair_lanes(p)) access_g<2>(p, idx, m, out, s);
@@ -1103,7 +1124,7 @@ void launch_tree_rank(const TreeQueryParams& p, const void* q, uint64_t m,
   } else if (p.quad.levels) {
     if (p.quad.nbase <= kQuadLdsBase) rank_quad<true>(p, qq, m, out, s);
     else rank_quad<false>(p, qq, m, out, s);
-  } else if (const int g = group_lanes(p, m, p.has_lines ? kGroup8Max : 0)) {
+  } else if (const int g = group_lanes(p, m, true)) {
     if (g == 16) rank_group<16>(p, qq, m, out, s);
     else rank_group<8>(p, qq, m, out, s);
   } else if (pair_lanes(p)) rank_g<2>(p, qq, m, out, s);

@@ -44,3 +44,27 @@ def test_short_batches(gpu, dt, sigma):
         assert np.array_equal(wt.select(wt.make_queries(cnt + 1, c)), np.full(sigma, n, np.uint64))
         assert np.array_equal(wt.select(wt.make_queries(np.zeros(sigma), c)),
                               np.full(sigma, n, np.uint64))
+
+
+@pytest.mark.parametrize("n", [(1 << 24) - 8, 1 << 24, (1 << 29) + 72])
+def test_short_batches_over_long_directories(gpu, n):
+    """Access and rank over the directory take 16 lanes per query from sizes
+    of batch and tree that the trees above do not have: batches around each
+    change of kernel, at the tree sizes around each."""
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(n)
+    period = 1_000_003  # the text repeats a block, so ranks are known
+    block = rng.integers(0, 256, period).astype(np.uint8)
+    text = np.resize(block, n)
+    prefix = np.zeros((256, period + 1), np.uint32)
+    for c in range(256):
+        prefix[c, 1:] = np.cumsum(block == c)
+    wt = WaveletTree(text, np.arange(256, dtype=np.uint8))
+    for m in (1, 127, 128, 512, 513, 4096, 4097, 8192, 8193):
+        at = rng.integers(0, n, m)
+        at[0] = n - 1
+        assert np.array_equal(wt.access(at.astype(np.uint64)), text[at]), m
+        at[0] = n
+        sym = rng.integers(0, 256, m)
+        want = at // period * prefix[sym, period].astype(np.int64) + prefix[sym, at % period]
+        assert np.array_equal(wt.rank(wt.make_queries(at, sym)), want.astype(np.uint64)), m
