@@ -662,23 +662,23 @@ __device__ __forceinline__ uint64_t level_rank_coop(const LevelView& v, uint64_t
   return Value ? ones : index - ones;
 }
 
-// position of the r-th (1-based) Value in the nw <= 15 words from w (the
-// first word's bits below off dropped), the words split over the group in
+// position of the r-th (1-based) Value in the Nw words from w (the first
+// word's bits below off dropped), the words split over the group in
 // contiguous shares; `none` when the words hold fewer than r
-template <int Value, int G>
-__device__ __forceinline__ uint64_t group_select_words(const uint64_t* w, uint32_t nw,
-                                                       uint32_t off, uint64_t r,
-                                                       uint64_t pos0, uint64_t none) {
-  constexpr uint32_t W = (15 + G - 1) / G;
+template <int Value, int G, uint32_t Nw>
+__device__ __forceinline__ uint64_t group_select_words(const uint64_t* w, uint32_t off,
+                                                       uint64_t r, uint64_t pos0,
+                                                       uint64_t none) {
+  constexpr uint32_t W = (Nw + G - 1) / G;  // words per lane
   const uint32_t t = group_lane<G>();
-  const uint32_t per = (nw + G - 1) / G, k0 = t * per;
+  const uint32_t k0 = t * W;
   uint64_t x[W];
   uint32_t cnt = 0;
 #pragma unroll
   for (uint32_t j = 0; j < W; ++j) {
     const uint32_t k = k0 + j;
     x[j] = 0;
-    if (j < per && k < nw) {
+    if (k < Nw) {
       x[j] = Value ? gld(w, k) : ~gld(w, k);
       if (k == 0) x[j] &= ~0ull << off;
     }
@@ -722,8 +722,8 @@ __device__ __forceinline__ uint64_t level_select_coop(const LevelView& v, uint64
         reinterpret_cast<const uint64_t*>(v.sel_lines + ((Value ? 0 : v.sel_zero_line) + jj) * 8);
     const uint64_t s = gld(lp, 0);
     const uint64_t r = jj ? i - jj * rate + 1 : i;
-    const uint64_t res = group_select_words<Value, G>(lp + 1, 15, static_cast<uint32_t>(s & 63),
-                                                      r, s & ~63ull, v.size);
+    const uint64_t res = group_select_words<Value, G, 15>(lp + 1, static_cast<uint32_t>(s & 63),
+                                                          r, s & ~63ull, v.size);
     if (res < v.size) return res;
   }
   const uint64_t j = i / kSampleRate;
@@ -747,28 +747,31 @@ __device__ __forceinline__ uint64_t level_select_coop(const LevelView& v, uint64
   if (k_lo < first) k_lo = first;
   if (k_hi > last) k_hi = last;
   // blocks k_lo + u (0 < u <= span) with fewer than r Values before them
-  // (the counts grow with u), counted by the lanes together.  Lane u's first
-  // entry, k_lo + u, is read beside the L1 entry, and the answer's entry
-  // comes from the lane that read it.
+  // (the counts grow with u), counted by the lanes together.  Each lane's
+  // first entry, u = 1 + its number, is read beside the L1 entry (from u = 0
+  // on, the 16 blocks between two samples of a half-full array took a group
+  // of 8 three turns), and the answer's entry comes from the lane that read
+  // it.
   const uint64_t span = k_hi - k_lo;
-  const uint32_t t = group_lane<G>();
-  const uint64_t e0 = t <= span ? gld(v.l2, k_lo + t) : 0;
+  const uint32_t u0 = group_lane<G>() + 1;  // a lane's first u
+  const uint64_t e0 = u0 <= span ? gld(v.l2, k_lo + u0) : 0;
   const uint64_t e1 = gld(v.l1, blk1);
   const uint64_t r = i - (Value ? e1 : (blk1 << 16) - e1);
   uint32_t below =
-      t != 0 && t <= span && (Value ? e0 : ((k_lo + t - first) << 9) - e0) < r ? 1u : 0u;
-  for (uint64_t u = t + G; u <= span; u += G) {
+      u0 <= span && (Value ? e0 : ((k_lo + u0 - first) << 9) - e0) < r ? 1u : 0u;
+  for (uint64_t u = u0 + G; u <= span; u += G) {
     const uint64_t k = k_lo + u;
     const uint64_t e = gld(v.l2, k);
     below += (Value ? e : ((k - first) << 9) - e) < r ? 1u : 0u;
   }
   const uint32_t at = group_sum<G>(below);
   const uint64_t blk2 = k_lo + at;
-  const uint32_t near = __shfl(static_cast<uint32_t>(e0), static_cast<int>(at % G), G);
-  const uint64_t e2 = at < G ? near : gld(v.l2, blk2);
+  const uint32_t by = at - 1;  // the lane whose first entry is the answer's (at = 0: none)
+  const uint32_t near = __shfl(static_cast<uint32_t>(e0), static_cast<int>(by % G), G);
+  const uint64_t e2 = by < G ? near : gld(v.l2, blk2);
   const uint64_t rr = r - (Value ? e2 : ((blk2 - first) << 9) - e2);
-  return group_select_words<Value, G>(reinterpret_cast<const uint64_t*>(v.words + (blk2 << 4)),
-                                      8, 0, rr, blk2 << 9, v.size);
+  return group_select_words<Value, G, 8>(
+      reinterpret_cast<const uint64_t*>(v.words + (blk2 << 4)), 0, rr, blk2 << 9, v.size);
 }
 
 // ---------------------------------------------------------------------------
