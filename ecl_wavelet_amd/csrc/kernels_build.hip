@@ -876,6 +876,25 @@ __device__ __forceinline__ uint32_t lds_bits32(const uint32_t* w, uint32_t x) {
   return __builtin_amdgcn_alignbit(w[(x >> 5) + 1], w[x >> 5], x & 31);
 }
 
+// What a build workgroup is told (quad_wg_one): kQuadWgFields counts and
+// positions of at most 40 bits, as in the line headers, in kQuadWgInfo words:
+// the low halves two to a word, then the high bytes together.
+constexpr uint32_t kQuadWgFields = 8;
+static_assert(kQuadWgInfo == kQuadWgFields / 2 + 1, "low halves, then a byte each");
+__device__ __forceinline__ void quad_wg_pack(uint64_t* o, const uint64_t (&f)[kQuadWgFields]) {
+  uint64_t high = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kQuadWgFields; j += 2) {
+    o[j / 2] = (f[j] & 0xFFFFFFFFull) | (f[j + 1] << 32);
+    high |= (f[j] >> 32 & 0xFFu) << (8 * j) | (f[j + 1] >> 32 & 0xFFu) << (8 * j + 8);
+  }
+  o[kQuadWgFields / 2] = high;
+}
+__device__ __forceinline__ uint64_t quad_wg_field(const uint64_t* o, uint32_t j) {
+  const uint64_t low = detail::gld(reinterpret_cast<const uint32_t*>(o), j);
+  return low | (detail::gld(o, kQuadWgFields / 2) >> (8 * j) & 0xFFu) << 32;
+}
+
 // Thread t takes the 4 words (128 positions) from word 4t of the
 // workgroup's range; a block scan of their ones gives every word's rank from
 // one directory rank at the range's start, and the node search runs once per
@@ -894,10 +913,10 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
   // start and end and a word past the end
   __shared__ uint32_t s_runs[kWords + 6];
   __shared__ uint32_t s_wave[4], s_wave13[4];
-  // from quad_wg_kernel: ones of level 2q before the range, the node holding
-  // its start (node0), node0's start and end, the ones of level 2q before
-  // node0 and the zeros in it, the digits 0, 1 and 2 before the range
-  __shared__ uint64_t s_info[kQuadWgInfo];
+  // from quad_wg_kernel: the node holding the range's start (node0), node0's
+  // start and end, the ones of level 2q before node0 and the zeros in it, the
+  // digits 0, 1 and 2 before the range
+  __shared__ uint64_t s_info[kQuadWgFields];
   __shared__ __align__(16) uint8_t s_lut[4096];
   reinterpret_cast<uint4*>(s_lut)[threadIdx.x] =
       detail::gld(reinterpret_cast<const uint4*>(qp.lut), threadIdx.x);
@@ -924,14 +943,16 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
   const uint32_t pc = __popc(a4[0]) + __popc(a4[1]) + __popc(a4[2]) + __popc(a4[3]);
   const uint32_t incl = detail::wave_incl_scan_u32(pc);
   if (lane == 63) s_wave[wave] = incl;
-  if (tid < kQuadWgInfo) s_info[tid] = detail::gld(qp.wg_info, blk * kQuadWgInfo + tid);
+  if (tid < kQuadWgFields) s_info[tid] = quad_wg_field(qp.wg_info + blk * kQuadWgInfo, tid);
   __syncthreads();
   uint32_t run0 = incl - pc;  // ones of the range before this thread's words
   for (uint32_t w = 0; w < wave; ++w) run0 += s_wave[w];
-  const uint64_t rank0 = s_info[0], node0 = s_info[1];
-  const uint64_t SN0 = s_info[2], SN10 = s_info[3], OB0 = s_info[4], ZN0 = s_info[5];
-  // the range's first position, its positions and the ones among them
+  const uint64_t node0 = s_info[0];
+  const uint64_t SN0 = s_info[1], SN10 = s_info[2], OB0 = s_info[3], ZN0 = s_info[4];
+  // the range's first position and the ones of level 2q before it (the digits
+  // 2 and 3), its positions and the ones among them
   const uint64_t Pr = 32 * k0;
+  const uint64_t rank0 = Pr - s_info[5] - s_info[6];
   const uint32_t len = Pr < n ? static_cast<uint32_t>(n - Pr < 32ull * nwords ? n - Pr : 32ull * nwords) : 0u;
   const uint32_t ones = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
   // one node: the zeros' run of level 2q + 1 starts at bit zx, the ones' at ox
@@ -1047,8 +1068,8 @@ __device__ __forceinline__ void quad_lines_wg(const QuadBuildParams& qp, uint64_
     const uint32_t w = 4 * tid + i, li = w / kQuadWordsPerLine;
     if (w < nwords && w == li * kQuadWordsPerLine) {
       const uint32_t d1 = run13 & 0xFFFFu, d3 = run13 >> 16;
-      const uint64_t c0 = s_info[6] + (32 * w - run - d1), c1 = s_info[7] + d1,
-                     c2 = s_info[8] + (run - d3);
+      const uint64_t c0 = s_info[5] + (32 * w - run - d1), c1 = s_info[6] + d1,
+                     c2 = s_info[7] + (run - d3);
       uint32_t* h = s_lines + li * 32;
       const uint64_t h0 = c0 | (c1 << 40);
       const uint64_t h1 = (c1 >> 24) | (c2 << 16);
@@ -1068,25 +1089,18 @@ __global__ __launch_bounds__(256) void quad_lines_kernel(QuadBuildParams qp) {
   quad_lines_wg(qp, blockIdx.x);
 }
 
-// Per build workgroup g (positions from P = 448 * 64 g): the ones of level
-// 2q before P, the node N holding P (the last position when P >= n), N's
-// start and end, the ones of level 2q before N and the zeros in N, and the
-// digits 0, 1 and 2 before P -- the chain of dependent loads (directory rank, node search, tables) that would
+// Per build workgroup g (positions from P = 448 * 64 g): the node N holding P
+// (the last position when P >= n), N's start and end, the ones of level 2q
+// before N and the zeros in N, and the digits 0, 1 and 2 before P -- the chain
+// of dependent loads (directory ranks, node search, tables) that would
 // otherwise hold up every build workgroup, here one thread each, all at once.
 __device__ __forceinline__ void quad_wg_one(const QuadBuildParams& qp, uint64_t g) {
   const uint64_t P = g * kQuadLinesPerWg * kQuadDigits;
   const uint64_t N = quad_node(qp.S, qp.nodes, P < qp.n ? P : qp.n - 1);
   auto cd = [&](uint64_t M, uint32_t d) { return detail::gld(qp.CD, 4 * M + d); };
-  uint64_t* o = qp.wg_info + g * kQuadWgInfo;
   const uint64_t r = detail::level_rank<1>(qp.a, P), SN = detail::gld(qp.S, N);
   const uint64_t n1 = cd(N + 1, 1) - cd(N, 1), ZN = (cd(N + 1, 0) - cd(N, 0)) + n1;
   const uint64_t OB = cd(N, 2) + cd(N, 3);
-  o[0] = r;
-  o[1] = N;
-  o[2] = SN;
-  o[3] = detail::gld(qp.S, N + 1);
-  o[4] = OB;
-  o[5] = ZN;
   // digits 0, 1, 2 before P: the node's before it (CD), plus its digits 1
   // and 3 up to P (the ones of level 2q + 1 in its two runs) and the rest of
   // its zeros and ones up to P
@@ -1094,9 +1108,10 @@ __device__ __forceinline__ void quad_wg_one(const QuadBuildParams& qp, uint64_t 
   const uint64_t rB = cd(N, 1) + cd(N, 3);  // ones of level 2q + 1 before S_N
   const uint64_t d1 = detail::level_rank<1>(qp.b, SN + zeros) - rB;
   const uint64_t d3 = detail::level_rank<1>(qp.b, SN + ZN + ones) - (rB + n1);
-  o[6] = cd(N, 0) + (zeros - d1);
-  o[7] = cd(N, 1) + d1;
-  o[8] = cd(N, 2) + (ones - d3);
+  const uint64_t f[kQuadWgFields] = {N, SN, detail::gld(qp.S, N + 1), OB, ZN,
+                                     cd(N, 0) + (zeros - d1), cd(N, 1) + d1,
+                                     cd(N, 2) + (ones - d3)};
+  quad_wg_pack(qp.wg_info + g * kQuadWgInfo, f);
 }
 __global__ __launch_bounds__(256) void quad_wg_kernel(QuadBuildParams qp, uint64_t nwg) {
   const uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;

@@ -29,3 +29,23 @@ def test_layout_workgroup_edges(gpu, n, sigma, layout):
     for c in (0, sigma // 3, sigma - 1):
         cs = np.full(len(at), c, dtype=np.uint64)
         assert np.array_equal(wt.rank(wt.make_queries(at, cs)), O.scan_rank_batch(text, at, cs))
+
+
+@pytest.mark.parametrize("sigma,lengths,fits", [(4, [448 * 64 * 300 - 1], 82573088),
+                                                (16, [448 * 64 * 150], 86837808),
+                                                (256, [1_000_000, 2_345_678], 97918880)])
+def test_forest_quad_layouts_memory_limit(gpu, sigma, lengths, fits):
+    """Free device memory that these texts' quad layouts have been accepted
+    with (lines, tables, 64 MiB to spare and 6 words of scratch per 64 quad
+    lines) stays enough for them."""
+    from ecl_wavelet_amd import DeviceBuffer, Forest, set_device_memory_cap
+    lengths = np.array(lengths, np.uint64)
+    starts = np.concatenate([[0], np.cumsum((lengths + 15) // 16 * 16)[:-1]]).astype(np.uint64)
+    text = (np.arange(int(starts[-1] + lengths[-1])) * 7 % sigma).astype(np.uint8)
+    d = DeviceBuffer.from_array(text)
+    forest = Forest(d, starts, lengths, np.full(len(lengths), sigma, np.uint64))
+    try:
+        set_device_memory_cap(0, fits)
+        forest.buildQuadLayouts()
+    finally:
+        set_device_memory_cap(0, 0)
