@@ -950,6 +950,9 @@ TreeMemory tree_memory(uint64_t n, uint64_t sigma, uint32_t L, int esize, bool h
                              ((n + 511) / 512) * 2 + ((n + 65535) / 65536) * 8 +
                              (n / 4096) * 8 + 64;
   const uint64_t tiles = n / pass_tile_codes(b.cw, 4) + 2 * sigma + 2;
+  // hist and excl rows; the last term is an upper bound's slack (the scan once
+  // kept a partial row per 256 tiles) and stays, so that what is reported and
+  // what is refused do not move
   const uint64_t scan = tiles * 256 * 12 + (tiles / 256 + 1) * 256 * 8;
   TreeMemory m;
   m.resident = per_level * L + scan + sigma * 64 + (n / 4096 + 4096) * 8 +

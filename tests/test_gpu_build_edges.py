@@ -39,6 +39,40 @@ def test_tile_and_chunk_edges(gpu, dt, sigma, kind):
         _check_structure_vs_oracle(wt, text, sigma)
 
 
+@pytest.mark.parametrize("kind", ["uniform", "rare", "sorted"])
+@pytest.mark.parametrize("dt,sigma", [(np.uint16, 65536), (np.uint32, 70000), (np.uint32, 1 << 17),
+                                      (np.uint64, 300), (np.uint64, 70000)])
+def test_later_passes_over_many_tiles(gpu, dt, sigma, kind):
+    """Two- and three-pass builds whose nodes span several tiles of every
+    pass, with codes that get narrower from pass to pass (4, 2, 1 bytes), and
+    8-byte alphabets."""
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(sigma)
+    for n in (4 * 32768 - 1, 6 * 32768 + 77):
+        text = _text(kind, n, sigma, rng).astype(dt)
+        wt = WaveletTree(text, np.arange(sigma, dtype=dt))
+        _check_structure_vs_oracle(wt, text, sigma)
+
+
+@pytest.mark.parametrize("span", [1, 2, 4])
+def test_span_edges(gpu, span):
+    """Text lengths around whole spans of tiles, where a workgroup's carried
+    words meet the next one's."""
+    from ecl_wavelet_amd import WaveletTree, set_build_span
+    rng = np.random.default_rng(span)
+    set_build_span(span)
+    try:
+        for dt, sigma in ((np.uint8, 4), (np.uint8, 20), (np.uint8, 256), (np.uint16, 1024)):
+            tile = 32768 // np.dtype(dt).itemsize
+            for n in (span * tile - 1, span * tile, span * tile + 1, 2 * span * tile + 31):
+                for kind in ("uniform", "rare"):
+                    text = _text(kind, n, sigma, rng).astype(dt)
+                    wt = WaveletTree(text, np.arange(sigma, dtype=dt))
+                    _check_structure_vs_oracle(wt, text, sigma)
+    finally:
+        set_build_span(0)
+
+
 @pytest.mark.parametrize("sigma", [4, 20, 75, 200])
 def test_mapped_bytes_edges(gpu, sigma):
     """Byte alphabets that are not 0..sigma-1 are mapped by table while the

@@ -65,6 +65,50 @@ def test_threads_and_released_buffers(gpu, tree):
     _check(tree, 1000, 5)
 
 
+def test_threads_over_two_trees_and_long_batches(gpu, tree):
+    """Callers at once on two trees of different element width, each with
+    batches of more chunks than slots (collected by a second thread) between
+    batches of one: the staging sets pass from tree to tree."""
+    from ecl_wavelet_amd import WaveletTree
+    rng = np.random.default_rng(21)
+    n = 200_003
+    alphabet = (np.arange(300) * 11 + 5).astype(np.uint32)
+    sym = rng.integers(0, 300, n)
+    wide_text = alphabet[sym]
+    wide = WaveletTree(wide_text, alphabet)
+    order = np.argsort(sym, kind="stable")
+    nth = np.empty(n, np.int64)
+    nth[order] = np.arange(n) - np.searchsorted(sym[order], np.arange(300))[sym[order]]
+
+    def check_wide(m, seed):
+        r = np.random.default_rng(seed)
+        at = r.integers(0, n, m)
+        assert np.array_equal(wide.access(at.astype(np.uint64)), wide_text[at])
+        got = wide.rank(wide.make_queries(at, wide_text[at]))
+        assert np.array_equal(got, nth[at].astype(np.uint64))
+        got = wide.select(wide.make_queries(nth[at] + 1, wide_text[at]))
+        assert np.array_equal(got, at.astype(np.uint64))
+
+    failed = []
+
+    def work(i):
+        try:
+            for m in (3 * CHUNK + 7 + i, 300 + i, 5 * CHUNK - i, 1):
+                if (i + m) % 2:
+                    _check(tree, m, 7 * i + m)
+                else:
+                    check_wide(m, 7 * i + m)
+        except BaseException as e:  # noqa: BLE001 - reported below
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed[0]
+
+
 @pytest.mark.parametrize("stage", ["directory", "query lines", "quad", "hex"])
 @pytest.mark.parametrize("dt", [np.uint8, np.uint16, np.uint64])
 def test_access_past_the_text_gives_zero(gpu, dt, stage):
