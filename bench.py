@@ -1186,7 +1186,7 @@ def main():
             "compulsory_bytes_per_launch": pb,
             "compulsory_gbps": compulsory,
             "compulsory_frac": compulsory / HBM_PEAK_GBPS,
-            "limiter": "LDS stores of the partition (the committed counter profile)",
+            "limiter": "VALU issue 0.71 and LDS 0.67 of the cycles, neither full (profiles/wt_pass_units.txt)",
             "launch_ms": pass_ms,
         },
     }

@@ -1017,6 +1017,8 @@ void rank_hex(const TreeQueryParams& p, const uint8_t* qq, uint64_t m, uint64_t*
 // 40, 16000 75 / 45 / 46, 30000 73 / 50 / 65 (one lane over hints 55, 51,
 // 47); over select lines 29.5 / 21 / 20, 30 / 23.5 / 27, 30 / 30 / 43.  Access
 // over query lines 15.1 / 11.5 / 10.9, 15.6 / 12 / 12.8, 16.5 / 14.6 / 19.5.
+// (The directory selects were faster still once a group of 8 took two turns
+// over a bracket: 8192 queries 30, 16384 34.)
 // With few levels the launch is most of the time and the lanes make no
 // difference (n = 5e7 over lines, 8192 queries, a pair and 16 lanes: sigma = 2
 // 5.5 / 5.5, sigma = 4 5.9 / 5.7, sigma = 20 10.2 / 7.6 us).

@@ -587,11 +587,14 @@ __global__ __launch_bounds__(256) void span_words_kernel(PassParams p) {
 // at one of two running addresses: about 40 VALU instructions per 16 codes
 // where a base, a rank and two counters per code took 140.  At n = 6e9, sigma
 // = 256 the pass went from 15.4 to 12.5 ms (94 -> 56 VALU instructions per
-// code).  What is left is the LDS: every ds_write of a wave takes 4.3 cycles
-// whatever its width, 5.6 with the partition's bank conflicts (measured over
-// 24 waves per CU), so the seven byte stores per code alone fill 60% of the
-// time.  Wider stores would have to be aligned: an unaligned ds_write_b16 or
-// b32 takes about 65 cycles.
+// code).  Neither unit is full now: of a CU's cycles VALU issue takes 0.71 and
+// the LDS 0.67 (a third of all cycles are bank conflicts), in phases between
+// barriers that do not overlap fully.  The seven byte stores per code are half
+// of the cycles at the 5.6 that a wave's store takes in the partition's
+// pattern (4.3 without conflicts, whatever its width); an unaligned
+// ds_write_b16 or b32 takes about 65.  Over two-byte codes, with twice the
+// chunks, VALU issue takes 0.81 and the LDS 0.48 (n = 5e8, 8 levels: 2.2 ms,
+// where one-byte codes take 1.3).
 //
 // Waves per SIMD that the tile's LDS allows (three, four, four workgroups
 // of eight waves per CU for 4, 2, 1 chunk rows): the register budget
