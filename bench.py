@@ -78,6 +78,7 @@ def parse():
                          "(n=6e9) and u16 sigma 2^16 Zipf(1.1) (n=2e9); 0 skips")
     ap.add_argument("--host-queries", type=int, default=100_000_000,
                     help="host-to-host section: queries per kind from host memory (0 skips)")
+    ap.add_argument("--detail", help="file for the result with every row and digit")
     ap.add_argument("--pmc-queries", action="store_true",
                     help="counter workload of the queries: the 1 GiB copy calibration, one "
                          "build, then the bench's access, rank and select batches once each")
@@ -200,10 +201,9 @@ def cpu_baseline(n, sigma, seed, args, sample):
     del text, B
     return {
         "value": 3.0 / (ta + tr + ts), "unit": "queries/s", "cores": threads, "kind": "port",
-        "sample": (f"variant A, the oracle's direct scans (OpenMP, {threads} threads) over the "
-                   f"same 6e9-symbol text, generated on the host: the first {len(idx)} access, "
-                   f"{len(r_a)} rank and {len(s_a)} select queries of the GPU's query arrays; "
-                   f"value = 1:1:1 mixed rate"),
+        "sample": (f"variant A, the oracle's direct scans (OpenMP) of the same text: the first "
+                   f"{len(idx)} access, {len(r_a)} rank and {len(s_a)} select queries of the "
+                   f"GPU's; value = 1:1:1 mixed rate"),
         "omp_threads": threads, "nproc": os.cpu_count(), "affinity_cpus": affinity,
         "access_qps": 1.0 / ta, "rank_qps": 1.0 / tr, "select_qps": 1.0 / ts,
         "rank_select_sample": len(r_a),
@@ -844,6 +844,53 @@ def run_queries(wt, timer, Q, d_idx, d_rq, d_sq, d_mq, d_out):
     return t
 
 
+# A reader that keeps only the last 8000 characters of the output still gets
+# the whole line.
+LINE_MAX = 8000
+SERVED_COLUMNS = ("rate_req_s", "p50_ms", "p99_ms", "queries_per_s")
+MATCHED_COLUMNS = ("p99_ms", "served_qps", "plain_qps")
+
+
+def result_line(res):
+    """The result as one line of JSON that fits LINE_MAX: numbers of 4 digits
+    (the headline value and its time in full), the rows of the serving and
+    full-size sweeps as lists with their names once under "columns", and of
+    the serving rates only those over the quad layouts; without the sections'
+    descriptions.  --detail writes everything."""
+    def short(x):
+        if isinstance(x, dict):
+            return {k: short(v) for k, v in x.items() if not k.endswith("_source")
+                    or k == "traffic_source"}
+        if isinstance(x, (list, tuple)):
+            return [short(v) for v in x]
+        if not isinstance(x, float):
+            return x
+        x = float(f"{x:.4g}")
+        return int(x) if abs(x) >= 1e5 else x
+
+    out = {k: v if k in ("value", "ms_per_step") else short(v) for k, v in res.items()}
+    for name in ("batched", "serving", "binary_rank_select", "host_to_host"):
+        if name in out:
+            out[name].pop("config", None)
+    sv = out.get("serving")
+    if sv:
+        sv.pop("p99_targets_ms", None)
+        for name, layout in sv.items():
+            del layout["plain"]
+            layout["matched_p99"] = [[r[c] for c in MATCHED_COLUMNS]
+                                     for r in layout["matched_p99"]]
+            rows = layout.pop("served")
+            if name == "quad":
+                layout["served"] = [[r[c] for c in SERVED_COLUMNS] for r in rows]
+        sv["columns"] = {"served": SERVED_COLUMNS, "matched_p99": MATCHED_COLUMNS}
+    sweep = out.get("full_size_sweep")
+    if sweep:
+        cols = list(sweep[0])
+        out["full_size_sweep"] = {"columns": cols,
+                                  "rows": [[r.get(c) for c in cols] for r in sweep]}
+    return json.dumps(out, separators=(",", ":"), ensure_ascii=False)
+
+
 def main():
     args = parse()
     if args.pmc_workload:
@@ -1094,12 +1141,10 @@ def main():
         "config": {
             "workload": (f"wavelet tree over a uint8 text of n={n} uniform over "
                          f"sigma={sigma} (device-resident); per step: 1 build, "
-                         f"{Q} each of access/rank/select + one mixed batch of {3 * Q} "
-                         f"over the plain directory, the query lines and select "
-                         f"lines, the same queries over them, then the quad lines and "
-                         f"quad select lines and the three kinds and the mixed batch over "
-                         f"them, then the hex lines and access, rank and the mixed batch "
-                         f"over them"),
+                         f"{Q} each of access/rank/select + a mixed batch of {3 * Q} "
+                         f"over the directory; the query and select lines, the quad and "
+                         f"quad select lines, the hex lines, and after each the same "
+                         f"queries over them (select not over hex lines)"),
             "n": n, "sigma": sigma, "queries_per_kind": Q, "levels": L,
         },
         "build_ms": build,
@@ -1180,9 +1225,8 @@ def main():
             "traffic": pass_traffic(n, sigma),
             "traffic_source": "profiles/wt_pass_counters_u8_n6e9_sigma256.txt",
             "bytes_per_launch": pab,
-            "bytes_basis": ("algorithmic: the level-at-a-time build's level reads, "
-                            "partition writes and bit writes, which this one pass "
-                            "replaces"),
+            "bytes_basis": ("algorithmic: a level-at-a-time build's level reads, partition "
+                            "and bit writes, which the pass replaces"),
             "compulsory_bytes_per_launch": pb,
             "compulsory_gbps": compulsory,
             "compulsory_frac": compulsory / HBM_PEAK_GBPS,
@@ -1205,7 +1249,13 @@ def main():
         res["full_size_sweep"] = bench_full_sweep(args)
     if not args.no_cpu:
         res["cpu_baseline"] = cpu_baseline(n, sigma, seed, args, sample)
-    print(json.dumps(res), flush=True)
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(res, f)
+    line = result_line(res)
+    if len(line) > LINE_MAX:
+        log(f"result line of {len(line)} characters")
+    print(line, flush=True)
 
 
 if __name__ == "__main__":
